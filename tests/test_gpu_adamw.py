@@ -106,6 +106,50 @@ def test_many_parameters_match_oracle(cfg, staged):
     assert opt.updates.value == ref.step_count.value and opt.pending.value == ref.pending.value
 
 
+@pytest.mark.parametrize("staged", [False, True])
+@pytest.mark.parametrize("cfg", [dict(lr=2e-3, weight_decay=0.01, clip_norm=0.5),
+                                 dict(lr=1e-3, accum_steps=2, clip_norm=1e-2)])
+def test_launch_tables_and_alignments_match_oracle(cfg, staged):
+    """260 parameters: past one elementwise table (70 rows), one norm table (240 of gradients alone,
+    160 with the accumulation buffers), many of them within one 128-value segment of a norm chunk,
+    others over several chunks; every second one a view at an odd offset, so its accesses go a value
+    at a time beside its neighbours' four. Bit for bit with the oracle's optimiser."""
+    from r9700training_amd.optim import DeviceAdamW, config
+    from oracle import oracle as O
+
+    print(f"case adamw tables {cfg} staged={staged}", flush=True)
+    rng = np.random.default_rng(5 + staged)
+    n = 260
+    sizes = [int(x) for x in rng.integers(1, 40, n)]
+    sizes[3], sizes[70], sizes[161], sizes[239], sizes[241] = 4095, 20000, 8192, 4097, 1028
+
+    def dev(a, i):
+        flat = torch.empty(a.size + 8, device="cuda")
+        at = 1 + i % 3 if i % 2 else 4
+        flat[at:at + a.size] = torch.tensor(a, device="cuda")
+        return flat[at:at + a.size]
+
+    w0 = [(0.1 * rng.standard_normal(k)).astype(np.float32) for k in sizes]
+    decay = [int(x) for x in rng.integers(0, 2, n)]
+    params = [dev(w, i) for i, w in enumerate(w0)]
+    outs = [torch.empty(k + 1, dtype=torch.bfloat16, device="cuda")[i % 2:][:k] for i, k in enumerate(sizes)]
+    opt = DeviceAdamW(params, config(**cfg), decay=decay, bf16_out=outs)
+    ref = O.AdamW(O.AdamWConfig.make(**cfg), [w.copy() for w in w0], decay=decay)
+    for s in range(4):
+        g = [rng.standard_normal(k).astype(np.float32) for k in sizes]
+        gd = [dev(x, i + s) for i, x in enumerate(g)]
+        assert opt.step(gd, staged=staged) == ref.step([_bf16_rounded(x) for x in g] if staged else g)
+        if staged:
+            torch.cuda.synchronize()
+            assert all(not x.any() for x in gd), "the staging buffers are cleared"
+    torch.cuda.synchronize()
+    for i in range(n):
+        for k, t, r in (("w", params[i], ref.w[i]), ("m", opt.m[i], ref.m[i]), ("v", opt.v[i], ref.v[i]),
+                        ("acc", opt.acc[i], ref.acc[i])):
+            assert np.array_equal(_bits(t), r.view(np.uint32)), (k, i)
+        assert torch.equal(outs[i].cpu(), params[i].cpu().to(torch.bfloat16)), i
+
+
 def test_step_refusals():
     from r9700training_amd import R97qError
     from r9700training_amd.optim import DeviceAdamW, config
