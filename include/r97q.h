@@ -413,7 +413,7 @@ int r97q_lora_shrink_q_bwd(int64_t T, int64_t K, const void* a, int32_t a_dtype,
  * buffers. The results are the reference host optimiser's bits: the same f32 operations in the
  * same order, the norm's double partials over the same 4096-element chunks added in chunk order.
  * No_decay names become decay = 0 on their parameters; the thread count has no counterpart.
- * An update is one elementwise launch over up to 16 parameters (two more with clipping); nothing
+ * An update is one elementwise launch over up to 70 parameters (two more with clipping); nothing
  * is read back to the host. */
 typedef struct {
     float lr, beta1, beta2, eps, weight_decay, clip_norm, lr_floor_frac;

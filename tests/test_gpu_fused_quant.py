@@ -77,6 +77,44 @@ def test_fused_matches_oracle(part, rows, n, group, dtype):
 
 
 @pytest.mark.parametrize("part", ["rmsnorm", "silu_mul", "sigmoid_mul"])
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("rows,n,group", [(3, 24, 8), (2, 1536, 512), (5, 768, 256), (2, 8704, 128), (1, 17408, 32),
+                                          (1, 24704, 128)])
+def test_lane_kernels_equal_the_general_ones(part, dtype, rows, n, group):
+    """Aligned bf16 / f32 calls with groups of 8 .. 512 columns hold the groups across lanes (the norm
+    one, two and three units a thread; 24704 columns are past its width); the same values in views one
+    element off take the general kernels. The gates are the same bits; the norm's row sums run in
+    another order, so its codes are the oracle's and its adjoint within the f32 rounding."""
+    from r9700training_amd.quant import fused_had_quant_i8g, fused_had_quant_i8g_bwd
+
+    print(f"case fused lanes {part} rows={rows} n={n} group={group} {dtype}", flush=True)
+    kw = KW[part]
+    rng, x0, x1, d0, d1 = _inputs(part, rows, n, dtype, 7 * n + group)
+
+    def off(t):
+        if t is None:
+            return None
+        return torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda")[1:].view(t.shape).copy_(t)
+
+    rnd = lambda shape: torch.tensor(rng.standard_normal(shape), dtype=torch.float32, device="cuda")  # noqa: E731
+    codes, scale, y = fused_had_quant_i8g(part, d0, d1, group, want_y=True, **kw)
+    codes_g, scale_g, y_g = fused_had_quant_i8g(part, off(d0), off(d1), group, want_y=True, **kw)
+    g, go, b0, b1 = rnd((rows, n)), rnd((rows, n)), rnd(tuple(d0.shape)), rnd((rows, n))
+    got = fused_had_quant_i8g_bwd(part, d0, d1, group, scale, g, go, dx0=b0.clone(), dx1=b1.clone(), **kw)
+    gen = fused_had_quant_i8g_bwd(part, off(d0), off(d1), group, scale, off(g), off(go), dx0=off(b0), dx1=off(b1), **kw)
+    torch.cuda.synchronize()
+    if part != "rmsnorm":
+        assert torch.equal(codes, codes_g) and torch.equal(scale, scale_g) and torch.equal(y, y_g)
+        assert torch.equal(got[0], gen[0]) and torch.equal(got[1], gen[1])
+    else:
+        assert torch.allclose(got[0], gen[0], rtol=4e-7, atol=float(4e-7 * gen[0].abs().max()))
+    wy, wc, ws = O.fused_quant(part, x0, x1, group, **kw)
+    assert np.array_equal(codes.cpu().numpy().astype(np.float64), wc)
+    assert np.array_equal(scale.cpu().numpy(), ws.astype(np.float32))
+    assert np.array_equal(y.view(torch.int16).cpu().numpy().view(np.uint16), _bf16_of(wy))
+
+
+@pytest.mark.parametrize("part", ["rmsnorm", "silu_mul", "sigmoid_mul"])
 def test_fused_mask_engaged(part):
     """A scale below the forward's (as a tape's cotangent may arrive against) clamps part of every
     group: the dropped elements must match the host rule |v / scale| > 127 exactly."""

@@ -76,6 +76,46 @@ def test_quant_saturated_group_on_the_card(rotated):
     assert np.allclose(d1.cpu().numpy()[0], want, rtol=1e-7, atol=0)
 
 
+@pytest.mark.parametrize("group", [4, 8, 16, 32, 64, 128, 256, 512, 1024])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_rotated_groups_equal_the_general_kernel(group, dtype):
+    """Rotated groups of 8 .. 512 columns are held across lanes when the buffers are aligned; the
+    same values in views one element off take the general kernel. Codes, scales and adjoint are the
+    same bits: rows of an odd number of groups, zeros, subnormals, infinities and NaN among the values,
+    and zero, infinite and NaN scales handed to the adjoint."""
+    from r9700training_amd.quant import quant_act_i8g, quant_act_i8g_bwd
+
+    print(f"case rotated groups {group} {dtype}", flush=True)
+    rng = np.random.default_rng(group)
+    rows, n = 7, 3 * group
+    a = (rng.standard_normal((rows, n)) * np.exp(3 * rng.standard_normal((rows, 1)))).astype(np.float32)
+    a[0, 0], a[1, group], a[2, :group], a[3, :] = np.inf, np.nan, 0.0, 1e-39
+    g = rng.standard_normal((rows, n)).astype(np.float32)
+    g[0, 1], g[1, 2], g[2, 3] = np.inf, np.nan, 1e-40
+
+    def off(t):  # the same values, one element past an aligned start
+        v = torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda")[1:].view(t.shape)
+        return v.copy_(t)
+
+    x = torch.tensor(a, device="cuda").to(dtype)
+    gd, dx0 = torch.tensor(g, device="cuda"), torch.randn((rows, n), device="cuda")
+    codes, scale = quant_act_i8g(x, group, True)
+    codes_g, scale_g = quant_act_i8g(off(x), group, True)
+    assert torch.equal(codes, codes_g)
+    assert torch.equal(scale.view(torch.int32), scale_g.view(torch.int32))
+    odd = scale.clone()
+    odd[4, 0], odd[5, 0], odd[6, 0] = 0.0, float("inf"), float("nan")
+    for s in (scale, odd):
+        dx = quant_act_i8g_bwd(x, s, gd, group, True, dx=dx0.clone())
+        dx_g = quant_act_i8g_bwd(off(x), s, off(gd), group, True, dx=off(dx0))
+        assert torch.equal(dx.isnan(), dx_g.isnan())
+        assert torch.equal(dx.nan_to_num(0.0, 1.0, -1.0), dx_g.nan_to_num(0.0, 1.0, -1.0))
+    finite = slice(4, rows)
+    want_codes, want_scale, _ = O.quant_act_i8g(x[finite].double().cpu().numpy(), group, True)
+    assert np.array_equal(codes[finite].cpu().numpy().astype(np.float64), want_codes)
+    assert np.array_equal(scale[finite].cpu().numpy(), want_scale.astype(np.float32))
+
+
 def test_quant_refusals():
     from r9700training_amd import R97qError
     from r9700training_amd.quant import quant_act_i8g
