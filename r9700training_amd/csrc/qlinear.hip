@@ -25,6 +25,7 @@
 #include "qlinear_fused.h"
 #include "qlinear_q.h"
 #include "qlinear_rt.h"
+#include "qlinear_sm.h"
 #include "status.h"
 
 #include <atomic>
@@ -44,6 +45,7 @@ struct Shape {
     int64_t T, N, K;
     int r;
     bool once;
+    bool small;  // the few-token path (qlinear_sm.h)
 };
 
 // The base products either decode each weight tile in the main loop, once for every 512-token
@@ -63,11 +65,24 @@ constexpr int64_t kDecodeOnceMinT = 32 * rt::kBM;          // any weight from 16
 constexpr int64_t kDecodeOnceMinTLarge = 16 * rt::kBM;     // weights of kDecodeOnceLarge values from 8192
 constexpr int64_t kDecodeOnceLarge = int64_t(1) << 23;
 std::atomic<int> g_decode_once{R97Q_DECODE_AUTO};
+// Whether a call takes the few-token path (qlinear_sm.h) where the choice is automatic: every call of at
+// most 128 tokens, and up to 1024 tokens while the products hold at most kSmWork steps of a
+// 128-token tile (16 for each CU) and a direction's partials stay within kSmPartBytes. Measured,
+// forward + backward, against the path for more tokens: 1 x 4096 x 4096 (tokens, outputs, inputs) 32 us
+// against 90, 128 x 1024 x 1024 25 against 71, 128 x 17408 x 5120 159 against 248, 256 x 4096 x 4096 76
+// against 105, 777 x 1408 x 2560 at rank 32 102 against 125, 1024 x 1024 x 1024 70 against 77; past
+// the line 300 x 4096 x 4096 at rank 32 (24 steps a CU) 123 against 118, 512 x 4096 x 4096 (32) 113 against
+// 106, 200 x 17408 x 5120 (85) 268 against 239.
+constexpr int64_t kSmAlwaysT = 128, kSmMaxT = 1024, kSmWork = 16 * 256, kSmPartBytes = int64_t(40) << 20;
+bool few_tokens(int64_t T, int64_t N, int64_t K) {
+    if (T <= 0 || T > kSmMaxT || T * (N > K ? N : K) * 4 > kSmPartBytes) return false;
+    return T <= kSmAlwaysT || (T + 127) / 128 * (N / kBN) * (K / rt::kStep) <= kSmWork;
+}
 Shape shape(int64_t T, int64_t N, int64_t K, int r) {
     const int m = g_decode_once.load(std::memory_order_relaxed);
     const bool once = m != R97Q_DECODE_AUTO ? m == R97Q_DECODE_ONCE
                                             : T >= kDecodeOnceMinT || (T >= kDecodeOnceMinTLarge && N * K >= kDecodeOnceLarge);
-    return Shape{T, N, K, r, once};
+    return Shape{T, N, K, r, once, m == R97Q_DECODE_AUTO && few_tokens(T, N, K)};
 }
 
 // Split-K of the fused kernel (rt::Params::ksplit, nfull). A launch holds tiles = ceil(T/512) x
@@ -210,6 +225,53 @@ BwdWs bwd_ws(const Shape& s) {
     return w;
 }
 
+// ---------------------------------------------------------------- the few-token path's layouts
+// The ranges the reduction of a product over T tokens is dealt over: about one workgroup a CU with
+// tiles of 32 and 64 tokens, two with 128 (measured at 4096 x 4096, forward + backward: at 32 tokens 256
+// workgroups 39 us, 512 46, 1024 69; at 128 tokens 65, 61, 89), two steps a range at least, and the
+// partials within kSmPartBytes
+int sm_ranges(int64_t T, int64_t outputs, int64_t red) {
+    const int64_t bm = sm::tile_tokens(T), tiles = (T + bm - 1) / bm * (outputs / kBN);
+    int64_t S = ((bm < 128 ? 256 : 512) + tiles - 1) / tiles;
+    const int64_t most = red / rt::kStep / 2, fit = kSmPartBytes / (T * outputs * 4);
+    S = S < most ? S : most;
+    S = S < fit ? S : fit;
+    return (int)(S < 1 ? 1 : S > 64 ? 64 : S);
+}
+
+// Forward: part [S, T, N] | tpart [SD, T, r] f32, and between the stage entries u [T, r] f32 (s.t) | act
+// [T, K] bf16 (X, as the tiled copy of the path for more tokens holds it).
+// Backward: part [S, T, K] | tpart [SD, T, r] f32, and between the stage entries u [T, r] (dt) | ts [T, r]
+// (s.t) f32 | Ac [r, K] bf16 | act [T, N] bf16 (dY). `fused`: the bytes without the stages' part.
+// the down product's ranges: one for few steps or many token blocks, up to a step a wave of its
+// workgroups (the finishing launch's workgroups each add the ranges, over every token)
+int sm_down_ranges(int64_t T, int64_t red) {
+    const int64_t waves = 8 * (T <= 128 ? 1 : (T + 127) / 128);
+    const int64_t n = (red / rt::kStep + waves - 1) / waves;
+    return (int)(n < 16 ? n : 16);
+}
+struct SmWs {
+    int S, SD;
+    int64_t part, tpart, u, ts, Ac, act, fused, total;
+};
+SmWs sm_ws(const Shape& s, bool fwd) {
+    SmWs w{};
+    const int64_t outs = fwd ? s.N : s.K;
+    w.S = sm_ranges(s.T, outs, fwd ? s.K : s.N);
+    w.SD = sm_down_ranges(s.T, fwd ? s.K : s.N);
+    w.tpart = align256((int64_t)w.S * s.T * outs * 4);
+    w.u = w.tpart + align256((int64_t)w.SD * s.T * s.r * 4);
+    w.ts = w.u + align256(s.T * s.r * 4);
+    w.Ac = w.ts + (fwd ? 0 : align256(s.T * s.r * 4));
+    w.act = w.Ac + (fwd ? 0 : align256((int64_t)s.r * s.K * 2));
+    w.fused = w.u;
+    w.total = w.act + align256(s.T * (fwd ? s.K : s.N) * 2);
+    return w;
+}
+
+int64_t fwd_total(const Shape& s) { return s.small ? sm_ws(s, true).total : fwd_ws(s).total; }
+int64_t bwd_total(const Shape& s) { return s.small ? sm_ws(s, false).total : bwd_ws(s).total; }
+
 // The adapter rows on their own (the shrink's and the expand's adjoints), workspace layouts:
 // shrink: P [T, 2r] | Pt [2r, ldt] | At [K, r] | part [chunks, r, K] | done
 // expand: Bt [rd, N] | Pt2 [2r, ldt] | part [chunks, r, N] | done
@@ -322,6 +384,150 @@ int check_ws(int64_t have, int64_t need, const void* ws, const char* who) {
         return R97Q_EWORKSPACE;
     }
     return R97Q_OK;
+}
+
+// ---------------------------------------------------------------- the few-token path
+// The first launch of a direction: the products (w non-null), the down product (rank > 0 and F non-null)
+int sm_products(const R97qWeight* w, bool fwd, const Shape& sh, const uint16_t* act, const uint16_t* F, uint8_t* wsb,
+                hipStream_t s) {
+    const SmWs ws = sm_ws(sh, fwd);
+    sm::Params p{};
+    p.w.T = sh.T;
+    p.w.N = sh.N;
+    p.w.K = sh.K;
+    p.act = act;
+    p.F = F;
+    p.rank = sh.r;
+    p.S = ws.S;
+    const int bm = sm::tile_tokens(sh.T);
+    p.mtiles = (int)((sh.T + bm - 1) / bm);
+    p.otiles = (int)((fwd ? sh.N : sh.K) / kBN);
+    p.SD = ws.SD;
+    p.mblocks = (int)((sh.T + 31) / 32);
+    p.ndown = sh.r > 0 && F ? p.mblocks * p.SD : 0;
+    p.nprod = w ? p.mtiles * p.otiles * p.S : 0;
+    p.part = reinterpret_cast<float*>(wsb + ws.part);
+    p.tpart = reinterpret_cast<float*>(wsb + ws.tpart);
+    if (p.ndown + p.nprod == 0) return R97Q_OK;
+    if (w) {
+        p.w.stream = w->stream;
+        p.w.scale_t = w->scale_t;
+        p.w.a24 = w->mad_a & 0xFFFFFFu;
+        p.w.b = w->mad_b;
+        p.w.run_rows = w->run_rows;
+    }
+    switch (w ? w->bits : R97Q_CODES8) {  // the down product alone reads no weight
+        case 3: sm::launch_products<3>(p, fwd, s); break;
+        case 4: sm::launch_products<4>(p, fwd, s); break;
+        case 5: sm::launch_products<5>(p, fwd, s); break;
+        case 6: sm::launch_products<6>(p, fwd, s); break;
+        default: sm::launch_products<R97Q_CODES8>(p, fwd, s); break;
+    }
+    return launch_status("sm_products_kernel");
+}
+
+// A finishing launch over u = the down product's ranges (staged: u as an earlier stage left it, `u` null
+// for rank 0)
+sm::Finish sm_finish(const Shape& sh, bool fwd, float scale, bool staged, uint8_t* wsb) {
+    const SmWs ws = sm_ws(sh, fwd);
+    sm::Finish f{};
+    f.T = sh.T;
+    f.rank = sh.r;
+    f.fwd = fwd;
+    f.U = reinterpret_cast<const float*>(wsb + (staged ? ws.u : ws.tpart));
+    f.SU = staged ? 1 : ws.SD;
+    f.scale = staged ? 1.0f : scale;
+    return f;
+}
+void sm_output(sm::Finish& f, const Shape& sh, bool fwd, const uint16_t* F, void* out, int32_t dtype, int32_t accumulate,
+               const uint8_t* wsb) {
+    const SmWs ws = sm_ws(sh, fwd);
+    f.part = reinterpret_cast<const float*>(wsb + ws.part);
+    f.S = ws.S;
+    f.outs = fwd ? sh.N : sh.K;
+    f.F = F;
+    f.out = out;
+    f.out_f32 = dtype == R97Q_F32;
+    f.accumulate = accumulate != 0;
+    f.vec = reinterpret_cast<uintptr_t>(out) % (f.out_f32 ? 16 : 8) == 0;
+}
+
+int sm_fwd(const R97qWeight* w, const Shape& sh, const uint16_t* X, const uint16_t* A, const uint16_t* B, float scale,
+           void* Y, int32_t y_dtype, float* t_out, uint8_t* wsb, hipStream_t s) {
+    if (int e = sm_products(w, true, sh, X, A, wsb, s)) return e;
+    sm::Finish f = sm_finish(sh, true, scale, false, wsb);
+    sm_output(f, sh, true, B, Y, y_dtype, 0, wsb);
+    f.t_out = t_out;
+    return sm::launch_finish(f, s);
+}
+int sm_fwd_prep(const Shape& sh, const uint16_t* X, const uint16_t* A, float scale, float* t_out, uint8_t* wsb,
+                hipStream_t s) {
+    if (int e = sm_products(nullptr, true, sh, X, A, wsb, s)) return e;
+    const SmWs ws = sm_ws(sh, true);
+    sm::Finish f = sm_finish(sh, true, scale, false, wsb);
+    f.t_out = t_out;
+    f.u_out = reinterpret_cast<float*>(wsb + ws.u);
+    f.copy[0] = {X, reinterpret_cast<uint16_t*>(wsb + ws.act), sh.T * sh.K};
+    return sm::launch_finish(f, s);
+}
+int sm_fwd_base(const R97qWeight* w, const Shape& sh, const uint16_t* B, void* Y, int32_t y_dtype, uint8_t* wsb,
+                hipStream_t s) {
+    const uint16_t* X = reinterpret_cast<const uint16_t*>(wsb + sm_ws(sh, true).act);
+    if (int e = sm_products(w, true, sh, X, nullptr, wsb, s)) return e;
+    sm::Finish f = sm_finish(sh, true, 1.0f, true, wsb);
+    sm_output(f, sh, true, B, Y, y_dtype, 0, wsb);
+    return sm::launch_finish(f, s);
+}
+
+int sm_bwd(const R97qWeight* w, const Shape& sh, const uint16_t* X, const uint16_t* dY, const uint16_t* A,
+           const uint16_t* B, float scale, const float* t, void* dX, int32_t dx_dtype, int32_t accumulate, float* dA,
+           float* dB, uint8_t* wsb, hipStream_t s) {
+    if (int e = sm_products(w, false, sh, dY, B, wsb, s)) return e;
+    sm::Finish f = sm_finish(sh, false, scale, false, wsb);
+    sm_output(f, sh, false, A, dX, dx_dtype, accumulate, wsb);
+    f.X = X;
+    f.K = sh.K;
+    f.dA = dA;
+    f.dY = dY;
+    f.t = t;
+    f.tscale = scale;
+    f.N = sh.N;
+    f.dB = dB;
+    return sm::launch_finish(f, s);
+}
+int sm_bwd_prep(const Shape& sh, const uint16_t* dY, const uint16_t* A, const uint16_t* B, const float* t, float scale,
+                uint8_t* wsb, hipStream_t s) {
+    if (int e = sm_products(nullptr, false, sh, dY, B, wsb, s)) return e;
+    const SmWs ws = sm_ws(sh, false);
+    sm::Finish f = sm_finish(sh, false, scale, false, wsb);
+    f.u_out = reinterpret_cast<float*>(wsb + ws.u);
+    f.t = t;
+    f.tscale = scale;
+    f.ts = reinterpret_cast<float*>(wsb + ws.ts);
+    f.copy[0] = {dY, reinterpret_cast<uint16_t*>(wsb + ws.act), sh.T * sh.N};
+    if (sh.r > 0) f.copy[1] = {A, reinterpret_cast<uint16_t*>(wsb + ws.Ac), (int64_t)sh.r * sh.K};
+    return sm::launch_finish(f, s);
+}
+int sm_bwd_grads(const Shape& sh, const uint16_t* X, const uint16_t* dY, float* dA, float* dB, uint8_t* wsb,
+                 hipStream_t s) {
+    sm::Finish f = sm_finish(sh, false, 1.0f, true, wsb);
+    f.X = X;
+    f.K = sh.K;
+    f.dA = dA;
+    f.dY = dY;
+    f.t = reinterpret_cast<const float*>(wsb + sm_ws(sh, false).ts);
+    f.tscale = 1.0f;
+    f.N = sh.N;
+    f.dB = dB;
+    return sm::launch_finish(f, s);
+}
+int sm_dx_base(const R97qWeight* w, const Shape& sh, void* dX, int32_t dx_dtype, int32_t accumulate, uint8_t* wsb,
+               hipStream_t s) {
+    const uint16_t* dY = reinterpret_cast<const uint16_t*>(wsb + sm_ws(sh, false).act);
+    if (int e = sm_products(w, false, sh, dY, nullptr, wsb, s)) return e;
+    sm::Finish f = sm_finish(sh, false, 1.0f, true, wsb);
+    sm_output(f, sh, false, reinterpret_cast<const uint16_t*>(wsb + sm_ws(sh, false).Ac), dX, dx_dtype, accumulate, wsb);
+    return sm::launch_finish(f, s);
 }
 
 // t = X.A^T (f32, kept for the backward), P = [hi | lo](s.t) in the forward workspace
@@ -591,11 +797,11 @@ int32_t r97q_set_decode_once(int32_t mode) {
 }
 
 int64_t r97q_fwd_workspace_bytes(int64_t T, int64_t N, int64_t K, int32_t rank) {
-    return fwd_ws(shape(T, N, K, rank)).total;
+    return fwd_total(shape(T, N, K, rank));
 }
 
 int64_t r97q_bwd_workspace_bytes(int64_t T, int64_t N, int64_t K, int32_t rank) {
-    return bwd_ws(shape(T, N, K, rank)).total;
+    return bwd_total(shape(T, N, K, rank));
 }
 
 int r97q_lora_fwd_prep(int64_t T, int64_t N, int64_t K, const uint16_t* X, const uint16_t* A,
@@ -610,8 +816,10 @@ int r97q_lora_fwd_prep(int64_t T, int64_t N, int64_t K, const uint16_t* X, const
         return R97Q_EINVAL;
     }
     const Shape sh = shape(T, N, K, rank);
-    if (int e = check_ws(workspace_bytes, fwd_ws(sh).total, workspace, who)) return e;
-    return fwd_prep(sh, X, A, scale, t_out, static_cast<uint8_t*>(workspace), (hipStream_t)stream);
+    if (int e = check_ws(workspace_bytes, fwd_total(sh), workspace, who)) return e;
+    uint8_t* wsb = static_cast<uint8_t*>(workspace);
+    if (sh.small) return sm_fwd_prep(sh, X, A, scale, t_out, wsb, (hipStream_t)stream);
+    return fwd_prep(sh, X, A, scale, t_out, wsb, (hipStream_t)stream);
 }
 
 int r97q_qlinear_fwd_base(const R97qWeight* w, const uint16_t* X, int64_t T, const uint16_t* B,
@@ -626,8 +834,10 @@ int r97q_qlinear_fwd_base(const R97qWeight* w, const uint16_t* X, int64_t T, con
         return R97Q_EINVAL;
     }
     const Shape sh = shape(T, w->rows, w->cols, rank);
-    if (int e = check_ws(workspace_bytes, fwd_ws(sh).total, workspace, who)) return e;
-    return fwd_base(w, sh, B, Y, y_dtype, static_cast<uint8_t*>(workspace), (hipStream_t)stream);
+    if (int e = check_ws(workspace_bytes, fwd_total(sh), workspace, who)) return e;
+    uint8_t* wsb = static_cast<uint8_t*>(workspace);
+    if (sh.small) return sm_fwd_base(w, sh, B, Y, y_dtype, wsb, (hipStream_t)stream);
+    return fwd_base(w, sh, B, Y, y_dtype, wsb, (hipStream_t)stream);
 }
 
 int r97q_qlinear_lora_fwd(const R97qWeight* w, const uint16_t* X, int64_t T, const uint16_t* A,
@@ -647,9 +857,10 @@ int r97q_qlinear_lora_fwd(const R97qWeight* w, const uint16_t* X, int64_t T, con
         return R97Q_EINVAL;
     }
     const Shape sh = shape(T, w->rows, w->cols, rank);
-    if (int e = check_ws(workspace_bytes, fwd_ws(sh).total, workspace, who)) return e;
+    if (int e = check_ws(workspace_bytes, fwd_total(sh), workspace, who)) return e;
     uint8_t* wsb = static_cast<uint8_t*>(workspace);
     const hipStream_t s = (hipStream_t)stream;
+    if (sh.small) return sm_fwd(w, sh, X, A, B, scale, Y, y_dtype, t_out, wsb, s);
     if (int e = fwd_prep(sh, X, A, scale, t_out, wsb, s)) return e;
     return fwd_base(w, sh, B, Y, y_dtype, wsb, s);
 }
@@ -668,8 +879,10 @@ int r97q_lora_bwd_prep(int64_t T, int64_t N, int64_t K, const uint16_t* dY, cons
         return R97Q_EINVAL;
     }
     const Shape sh = shape(T, N, K, rank);
-    if (int e = check_ws(workspace_bytes, bwd_ws(sh).total, workspace, who)) return e;
-    return bwd_prep(sh, dY, A, B, t, scale, static_cast<uint8_t*>(workspace), (hipStream_t)stream);
+    if (int e = check_ws(workspace_bytes, bwd_total(sh), workspace, who)) return e;
+    uint8_t* wsb = static_cast<uint8_t*>(workspace);
+    if (sh.small) return sm_bwd_prep(sh, dY, A, B, t, scale, wsb, (hipStream_t)stream);
+    return bwd_prep(sh, dY, A, B, t, scale, wsb, (hipStream_t)stream);
 }
 
 int r97q_lora_bwd_grads(int64_t T, int64_t N, int64_t K, const uint16_t* X, const uint16_t* dY,
@@ -685,8 +898,10 @@ int r97q_lora_bwd_grads(int64_t T, int64_t N, int64_t K, const uint16_t* X, cons
         return R97Q_EINVAL;
     }
     const Shape sh = shape(T, N, K, rank);
-    if (int e = check_ws(workspace_bytes, bwd_ws(sh).total, workspace, who)) return e;
-    return bwd_grads(sh, X, dY, dA, dB, static_cast<uint8_t*>(workspace), (hipStream_t)stream);
+    if (int e = check_ws(workspace_bytes, bwd_total(sh), workspace, who)) return e;
+    uint8_t* wsb = static_cast<uint8_t*>(workspace);
+    if (sh.small) return sm_bwd_grads(sh, X, dY, dA, dB, wsb, (hipStream_t)stream);
+    return bwd_grads(sh, X, dY, dA, dB, wsb, (hipStream_t)stream);
 }
 
 int r97q_qlinear_dx_base(const R97qWeight* w, const uint16_t* dY, int64_t T, int32_t rank, void* dX,
@@ -701,8 +916,10 @@ int r97q_qlinear_dx_base(const R97qWeight* w, const uint16_t* dY, int64_t T, int
         return R97Q_EINVAL;
     }
     const Shape sh = shape(T, w->rows, w->cols, rank);
-    if (int e = check_ws(workspace_bytes, bwd_ws(sh).total, workspace, who)) return e;
-    return dx_base(w, sh, dX, dx_dtype, dx_accumulate, static_cast<uint8_t*>(workspace), (hipStream_t)stream);
+    if (int e = check_ws(workspace_bytes, bwd_total(sh), workspace, who)) return e;
+    uint8_t* wsb = static_cast<uint8_t*>(workspace);
+    if (sh.small) return sm_dx_base(w, sh, dX, dx_dtype, dx_accumulate, wsb, (hipStream_t)stream);
+    return dx_base(w, sh, dX, dx_dtype, dx_accumulate, wsb, (hipStream_t)stream);
 }
 
 int r97q_qlinear_lora_bwd(const R97qWeight* w, const uint16_t* X, const uint16_t* dY, int64_t T,
@@ -723,9 +940,12 @@ int r97q_qlinear_lora_bwd(const R97qWeight* w, const uint16_t* X, const uint16_t
         return R97Q_EINVAL;
     }
     const Shape sh = shape(T, w->rows, w->cols, rank);
-    if (int e = check_ws(workspace_bytes, bwd_ws(sh).total, workspace, who)) return e;
+    if (int e = check_ws(workspace_bytes, bwd_total(sh), workspace, who)) return e;
     uint8_t* wsb = static_cast<uint8_t*>(workspace);
     const hipStream_t s = (hipStream_t)stream;
+    if (sh.small)
+        return sm_bwd(w, sh, X, dY, A, B, scale, t, dX, dx_dtype, dx_accumulate, rank > 0 ? dA : nullptr,
+                      rank > 0 ? dB : nullptr, wsb, s);
     if (int e = bwd_prep(sh, dY, A, B, t, scale, wsb, s)) return e;
     // the factor gradients' chunk sums by the gradient launch, added into dA and dB by the dX
     // launch (spread over its workgroups, in chunk order)
@@ -964,7 +1184,9 @@ int r97q_qlinear_lora_fwd_noalloc(const R97qWeight* w, const uint16_t* X, int64_
         return R97Q_EINVAL;
     }
     const Shape sh = shape(T, w->rows, w->cols, rank);
-    const int64_t need = fwd_ws(sh, true).total;
+    // the few-token path's layout fits the array (kSmPartBytes); the others' runs the fused kernel
+    const bool small = sh.small && sm_ws(sh, true).fused <= kNoAllocScratchBytes;
+    const int64_t need = small ? sm_ws(sh, true).fused : fwd_ws(sh, true).total;
     if (need > kNoAllocScratchBytes) {
         set_error("%s: T %lld x K %lld at rank %d needs %lld workspace bytes, past the %lld this entry holds "
                   "(use r97q_qlinear_lora_fwd with a workspace)",
@@ -974,6 +1196,7 @@ int r97q_qlinear_lora_fwd_noalloc(const R97qWeight* w, const uint16_t* X, int64_
     uint8_t* wsb = nullptr;
     if (int e = scratch_of_current_device(&wsb, who)) return e;
     const hipStream_t s = (hipStream_t)stream;
+    if (small) return sm_fwd(w, sh, X, A, B, scale, Y, y_dtype, t_out, wsb, s);
     if (int e = fwd_prep(sh, X, A, scale, t_out, wsb, s)) return e;
     return fwd_base(w, sh, B, Y, y_dtype, wsb, s, true);
 }

@@ -1,0 +1,137 @@
+"""The few-token path (csrc/qlinear_sm.h): at most 128 tokens, or 1024 while the products are small, the
+layer's forward and backward run as two launches each, the products' reductions dealt over ranges.
+
+At the edges of its tiles (32, 64, 128 tokens) and ranges, over the weight forms, ranks, output types and
+an unaligned output, it is held to the path for more tokens (R97Q_DECODE_FUSED asks for it): the decoded
+weights are the same bf16 values and every product is exact in f32, so the two differ by the order of f32
+sums of K or N terms and by the [hi | lo] bf16 split (16 bits) of the adapter's activations there --
+2e-5 relative, and a bf16 output by its own rounding (2^-8). Values against the float64 host rows are
+tests/test_gpu_qlinear.py's (its cases run this path too)."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+import iqr_synth as S
+from gpu_util import bf16_tensor, device_desc, prepared
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def modes():
+    from r9700training_amd import R97Q_DECODE_AUTO, R97Q_DECODE_FUSED, lib
+
+    L = lib()
+    yield lambda few: L.r97q_set_decode_once(R97Q_DECODE_AUTO if few else R97Q_DECODE_FUSED)
+    assert L.r97q_set_decode_once(R97Q_DECODE_AUTO) >= 0
+
+
+def _weight(N, K, bits, run, codes8, seed, keep):
+    from r9700training_amd.qlinear import QWeight
+
+    rng = np.random.default_rng(seed)
+    p = S.trellis(rows=N, cols=K, bits=bits, run_rows=run, rowf=True, seed=seed, packed=True,
+                  scale_col=(0.75 + 0.5 * rng.random(K // 128)).astype(np.float32))
+    if not codes8:
+        return prepared(p, keep)
+    sc = torch.from_numpy(p.scale_col).cuda()
+    keep.append(sc)
+    return QWeight(device_desc(p, keep), scale_col=sc, codes8=True)
+
+
+def _rel(a, b):
+    return float((a.double() - b.double()).norm() / b.double().norm())
+
+
+CASES = [
+    # T, N, K, r, bits, run, codes8, bf16 out
+    (1, 128, 128, 0, 5, 128, False, False),     # one range of two steps
+    (1, 384, 2048, 16, 5, 256, False, True),    # a short last run, many ranges
+    (31, 512, 640, 8, 3, 64, False, False),
+    (32, 640, 512, 64, 4, 96, False, False),
+    (33, 256, 384, 32, 6, 32, False, True),
+    (64, 1024, 256, 16, 5, 256, True, False),
+    (65, 128, 1152, 64, 6, 128, False, False),
+    (128, 384, 384, 8, 4, 256, False, False),
+    (129, 512, 768, 16, 5, 256, False, True),   # past the unconditional line, two token tiles
+    (500, 640, 896, 64, 5, 128, True, False),
+    (1024, 256, 512, 32, 3, 256, False, False),  # the most tokens
+]
+
+
+@pytest.mark.parametrize("T,N,K,r,bits,run,codes8,bf16", CASES)
+def test_few_tokens_match_the_other_path(modes, T, N, K, r, bits, run, codes8, bf16):
+    from r9700training_amd.qlinear import qlinear_lora_bwd, qlinear_lora_fwd
+
+    print(f"case few tokens T={T} N={N} K={K} r={r} bits={bits} codes8={codes8} bf16={bf16}", flush=True)
+    rng = np.random.default_rng(T + N + K)
+    keep = []
+    w = _weight(N, K, bits, run, codes8, T + bits, keep)
+    X, dY = bf16_tensor(rng.standard_normal((T, K))), bf16_tensor(rng.standard_normal((T, N)))
+    A = bf16_tensor(0.01 * rng.standard_normal((r, K))) if r else None
+    B = bf16_tensor(0.01 * rng.standard_normal((N, r))) if r else None
+    dt = torch.bfloat16 if bf16 else torch.float32
+    base = torch.randn((T, K), device="cuda").to(dt)
+    got = {}
+    for few in (True, False):
+        modes(few)
+        # outputs one element past an aligned start take the value-by-value stores
+        y = torch.empty(T * N + 1, dtype=dt, device="cuda")[few:][: T * N].view(T, N)
+        dx = torch.empty(T * K + 1, dtype=dt, device="cuda")[few:][: T * K].view(T, K).copy_(base)
+        Y, t = qlinear_lora_fwd(w, X, A, B, 2.0, out=y)
+        Y2, _ = qlinear_lora_fwd(w, X, A, B, 2.0, y_dtype=dt)
+        assert torch.equal(Y, Y2)
+        dA = torch.ones((r, K), device="cuda") if r else None
+        dB = torch.ones((N, r), device="cuda") if r else None
+        dX, dA, dB = qlinear_lora_bwd(w, X, dY, A, B, t, 2.0, dX=dx, accumulate=True, dA=dA, dB=dB)
+        dX2, dA2, dB2 = qlinear_lora_bwd(w, X, dY, A, B, t, 2.0, dX=base.clone(), accumulate=True)
+        assert torch.equal(dX, dX2)
+        if r:
+            assert torch.allclose(dA, dA2 + 1) and torch.allclose(dB, dB2 + 1)
+        got[few] = (Y, dX) if not r else (Y, dX, t, dA2, dB2)
+    torch.cuda.synchronize()
+    for i, (a, b) in enumerate(zip(got[True], got[False])):
+        e = _rel(a, b)
+        assert torch.isfinite(a).all() and e <= (2 ** -8 if bf16 and i < 2 else 2e-5), (i, e)
+
+
+@pytest.mark.parametrize("T,N,K,r", [(7, 384, 512, 16), (130, 256, 384, 0), (300, 512, 256, 64)])
+def test_stages_keep_their_operands(T, N, K, r):
+    """The stage entries on this path: the fused entries' bits, with X and dY overwritten between the
+    preparation and the product (the preparation holds them, as it holds the tiled copy on the path
+    for more tokens), and the forward that allocates nothing the same bits."""
+    from r9700training_amd import R97Q_F32, _ptr, _stream, check, lib
+    from r9700training_amd.qlinear import bwd_workspace, fwd_workspace, qlinear_lora_bwd, qlinear_lora_fwd
+
+    print(f"case few tokens stages T={T} N={N} K={K} r={r}", flush=True)
+    rng = np.random.default_rng(T)
+    keep = []
+    w = _weight(N, K, 5, 128, False, T, keep)
+    X, dY = bf16_tensor(rng.standard_normal((T, K))), bf16_tensor(rng.standard_normal((T, N)))
+    A = bf16_tensor(0.01 * rng.standard_normal((r, K))) if r else None
+    B = bf16_tensor(0.01 * rng.standard_normal((N, r))) if r else None
+    Y, t = qlinear_lora_fwd(w, X, A, B, 2.0, y_dtype=torch.float32)
+    dX, dA, dB = qlinear_lora_bwd(w, X, dY, A, B, t, 2.0, dx_dtype=torch.float32)
+    L, P, st = lib(), _ptr, _stream()
+    ws, wb = fwd_workspace(T, N, K, r), bwd_workspace(T, N, K, r)
+    Ys, dXs = torch.empty_like(Y), torch.empty_like(dX)
+    ts = torch.empty_like(t) if r else None
+    x, g = X.clone(), dY.clone()
+    check(L.r97q_lora_fwd_prep(T, N, K, P(x), P(A), r, 2.0, P(ts), P(ws), ws.numel(), st), "fwd_prep")
+    x.fill_(float("nan"))
+    check(L.r97q_qlinear_fwd_base(C.byref(w.w), P(x), T, P(B), r, P(Ys), R97Q_F32, P(ws), ws.numel(), st), "fwd_base")
+    check(L.r97q_lora_bwd_prep(T, N, K, P(g), P(A), P(B), P(t), r, 2.0, P(wb), wb.numel(), st), "bwd_prep")
+    dAs = torch.zeros_like(dA) if r else None
+    dBs = torch.zeros_like(dB) if r else None
+    check(L.r97q_lora_bwd_grads(T, N, K, P(X), P(g), r, P(dAs), P(dBs), P(wb), wb.numel(), st), "bwd_grads")
+    g.fill_(float("nan"))
+    check(L.r97q_qlinear_dx_base(C.byref(w.w), P(g), T, r, P(dXs), R97Q_F32, 0, P(wb), wb.numel(), st), "dx_base")
+    Yn = torch.empty_like(Y)
+    tn = torch.empty_like(t) if r else None
+    check(L.r97q_qlinear_lora_fwd_noalloc(C.byref(w.w), P(X), T, P(A), P(B), r, 2.0, P(Yn), R97Q_F32, P(tn), st), "noalloc")
+    torch.cuda.synchronize()
+    assert torch.equal(Y, Ys) and torch.equal(dX, dXs) and torch.equal(Y, Yn)
+    if r:
+        assert torch.equal(t, ts) and torch.equal(dA, dAs) and torch.equal(dB, dBs) and torch.equal(t, tn)
