@@ -66,20 +66,18 @@ int down_rank(int r);          // r rounded up to a multiple of 16
 int64_t grad_ld(int64_t T);    // the transposed splits' row length: T rounded up to 64
 int64_t grad_blocks(int64_t C);  // the gradient launch's column blocks over C columns (its counters)
 // the gradient launch's token chunks (at most this many) and their length in tokens, for dA over K
-// columns and dB over N
-int64_t grad_chunks(int64_t T, int64_t K, int64_t N);
-int64_t grad_chunk_rows(int64_t T, int64_t K, int64_t N);
+// columns and dB over N at rank r
+int64_t grad_chunks(int64_t T, int64_t K, int64_t N, int r);
+int64_t grad_chunk_rows(int64_t T, int64_t K, int64_t N, int r);
 
 int launch_lora_down(const DownArgs& a, hipStream_t s);
 int launch_lora_grads(int r, const GradArgs& g, int nz, hipStream_t s);
 // dst = the fused kernels' tiled copy (act_tiles.h) of act [T, R] bf16 (R a multiple of 64)
 int launch_act_tile(const uint16_t* act, int64_t T, int64_t R, uint16_t* dst, hipStream_t s);
-int launch_transpose2(const uint16_t* B, uint16_t* Bt, int64_t N, const uint16_t* A, uint16_t* At,
-                      int64_t K, int r, hipStream_t s);
 // P [T, 2r] / Pt [2r, ldt] = [hi | lo](scale * U), U f32 [T, r]; either output may be null;
-// zero [nzero] = 0 (a following gradient launch's counters)
+// zero [nzero] = 0 (a following gradient launch's counters); At [K, r] = A^T, A [r, K] (null: none)
 int launch_split(const float* U, int64_t T, int r, int64_t ldt, float scale, uint16_t* P, uint16_t* Pt,
-                 int* zero, int nzero, hipStream_t s);
+                 int* zero, int nzero, const uint16_t* A, uint16_t* At, int64_t K, hipStream_t s);
 // the coded activation (codes [T, K]: int8, or f32 code values when code_f32; f32 scale a_scale
 // [T, groups], group width gw):
 //   da [T, K] += g * a_scale;  ds [T, groups] += sum over each group of g * code  (g f32 [T, K];

@@ -22,11 +22,10 @@
 //                      chunk of a column block to finish adds them into dA or dB in chunk order
 //                      (deterministic; the leaves are added into, as the reference's rows add
 //                      into the step's f32 gradients).
-//   split_kernel       an f32 [T, r] operand (a cotangent handed in) -> its [hi | lo] splits.
+//   split_kernel       an f32 [T, r] operand (a cotangent handed in) -> its [hi | lo] splits, and
+//                      A [r, K] -> A^T [K, r] beside it.
 //   lora_up_kernel     the up-projection t_cot . A of the shrink's adjoint, on its own (the fused
 //                      dX kernel carries it in its epilogue when the base product runs too).
-//   transpose2_kernel  B [N, r] -> B^T [rd, N] (zero rows up to the 16-wide rank) and
-//                      A [r, K] -> A^T [K, r], in one launch.
 //   coded_cot_kernel   the coded shrink's two cotangents from the value-space one g = t_cot . A:
 //                      the code's g * scale and the scale's sum over its group of g * code.
 //   coded_x_kernel     the coded activation's values x = code * scale as a [hi | lo] bf16 pair (the
@@ -609,11 +608,17 @@ __global__ __launch_bounds__(512) void lora_grads_kernel(GradArgs ga) {
 
 // ---------------------------------------------------------------- split and up
 // P [T, 2r] = [hi | lo](s * U[m][j]) row-major, Pt [2r, ldt] the same transposed (zero for
-// T <= m < ldt). One thread an (m, j), m < ldt.
+// T <= m < ldt). One thread an (m, j), m < ldt. At [K, r] = A^T beside it (blockIdx.y 1; null: none).
 __global__ __launch_bounds__(256) void split_kernel(const float* __restrict__ U, int64_t T, int r, int64_t ldt,
                                                     float s, uint16_t* __restrict__ P, uint16_t* __restrict__ Pt,
-                                                    int* __restrict__ zero, int nzero) {
+                                                    int* __restrict__ zero, int nzero,
+                                                    const uint16_t* __restrict__ A, uint16_t* __restrict__ At,
+                                                    int64_t K) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (blockIdx.y == 1) {
+        if (i < (int64_t)r * K) At[i] = A[(i % r) * K + i / r];
+        return;
+    }
     if (i < nzero) zero[i] = 0;
     if (i >= ldt * r) return;
     const int64_t m = i / r;
@@ -750,25 +755,6 @@ __global__ __launch_bounds__(256) void act_tile_kernel(const uint16_t* __restric
     *reinterpret_cast<uint4*>(dst + ((s * (int64_t)gridDim.y + rb) * 4 + (c & 3)) * 512 + (32 * (c >> 2) + i) * 8) = v;
 }
 
-// ---------------------------------------------------------------- transposes
-// y 0: Bt[q][n] = B[n][q] for q < r, 0 for r <= q < rd;  y 1: At[k][j] = A[j][k]
-__global__ __launch_bounds__(256) void transpose2_kernel(const uint16_t* __restrict__ B,
-                                                         uint16_t* __restrict__ Bt, int64_t N,
-                                                         const uint16_t* __restrict__ A,
-                                                         uint16_t* __restrict__ At, int64_t K, int r,
-                                                         int rd) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (blockIdx.y == 0) {
-        if (i >= (int64_t)rd * N) return;
-        const int64_t q = i / N, n = i % N;
-        Bt[i] = q < r ? B[n * r + q] : (uint16_t)0;
-    } else {
-        if (i >= (int64_t)r * K) return;
-        const int64_t k = i / r, j = i % r;
-        At[i] = A[j * K + k];
-    }
-}
-
 template <int RD>
 int down_r(const DownArgs& a, hipStream_t s) {
     const int nw = a.Kin % 256 == 0 ? kDownWavesMax : 4;
@@ -823,17 +809,21 @@ int launch_lora_down(const DownArgs& a, hipStream_t s) {
 
 int64_t grad_blocks(int64_t C) { return (C + kGradCols - 1) / kGradCols; }
 
-int64_t grad_chunks(int64_t T, int64_t K, int64_t N) {
-    // about 256 workgroups (one a CU) over dA's and dB's column blocks
+int64_t grad_chunks(int64_t T, int64_t K, int64_t N, int r) {
+    // Workgroups for the CUs over dA's and dB's column blocks, rounded down: one more than a CU holds at a
+    // time makes the launch twice as long for the CU that takes it (dB over 12288 columns and 4096
+    // tokens at rank 16: 5 chunks, 240 workgroups, 31 us; 6 chunks, 288, 46). One workgroup a CU (two
+    // measured slower at ranks 8 to 32, 27-40%: the chunks' partial sums), two at rank 64, whose tiles
+    // are half as long (2048 + 8192 columns, 16384 tokens: 12 chunks 114 us, 6 chunks 130).
     const int64_t cols = grad_blocks(K) + grad_blocks(N);
-    int64_t chunks = (256 + cols - 1) / cols;
+    int64_t chunks = (r == 64 ? 512 : 256) / cols;
     const int64_t tiles = grad_ld(T) / 64;  // no chunk smaller than one 64-token tile
     if (chunks > tiles) chunks = tiles;
     return chunks < 1 ? 1 : chunks;
 }
 
-int64_t grad_chunk_rows(int64_t T, int64_t K, int64_t N) {
-    const int64_t chunks = grad_chunks(T, K, N);
+int64_t grad_chunk_rows(int64_t T, int64_t K, int64_t N, int r) {
+    const int64_t chunks = grad_chunks(T, K, N, r);
     const int64_t ldt = grad_ld(T);
     return ((ldt + chunks - 1) / chunks + 63) / 64 * 64;  // whole 64-token tiles
 }
@@ -856,10 +846,11 @@ int launch_lora_grads(int r, const GradArgs& g, int nz, hipStream_t s) {
 }
 
 int launch_split(const float* U, int64_t T, int r, int64_t ldt, float scale, uint16_t* P, uint16_t* Pt,
-                 int* zero, int nzero, hipStream_t s) {
-    const int64_t n = ldt * r > nzero ? ldt * r : nzero;
-    hipLaunchKernelGGL(split_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, U, T, r, ldt, scale, P,
-                       Pt, zero, nzero);
+                 int* zero, int nzero, const uint16_t* A, uint16_t* At, int64_t K, hipStream_t s) {
+    int64_t n = ldt * r > nzero ? ldt * r : nzero;
+    if (At && r * K > n) n = r * K;
+    hipLaunchKernelGGL(split_kernel, dim3((unsigned)((n + 255) / 256), At ? 2 : 1), dim3(256), 0, s, U, T, r, ldt,
+                       scale, P, Pt, zero, nzero, A, At, K);
     return launch_status("split_kernel");
 }
 
@@ -902,15 +893,6 @@ int launch_act_tile(const uint16_t* act, int64_t T, int64_t R, uint16_t* dst, hi
     hipLaunchKernelGGL(act_tile_kernel, dim3((unsigned)(R / 64), (unsigned)((T + 31) / 32)), dim3(256), 0, s, act, T,
                        R, dst);
     return launch_status("act_tile_kernel");
-}
-
-int launch_transpose2(const uint16_t* B, uint16_t* Bt, int64_t N, const uint16_t* A, uint16_t* At,
-                      int64_t K, int r, hipStream_t s) {
-    const int rd = down_rank(r);
-    const int64_t n = (int64_t)rd * N > (int64_t)r * K ? (int64_t)rd * N : (int64_t)r * K;
-    hipLaunchKernelGGL(transpose2_kernel, dim3((unsigned)((n + 255) / 256), 2), dim3(256), 0, s, B, Bt, N, A,
-                       At, K, r, rd);
-    return launch_status("transpose2_kernel");
 }
 
 }  // namespace r97q

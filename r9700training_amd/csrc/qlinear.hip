@@ -215,8 +215,8 @@ BwdWs bwd_ws(const Shape& s) {
     w.PtA = w.P + align256(s.T * 2 * s.r * 2);
     w.PtB = w.PtA + align256(2 * s.r * ldt * 2);
     // the chunk partials of either factor's gradient: as many as its launch alone takes (the most)
-    const int64_t chunksA = grad_chunks(s.T, s.K, 0);
-    const int64_t chunksB = grad_chunks(s.T, 0, s.N);
+    const int64_t chunksA = grad_chunks(s.T, s.K, 0, s.r);
+    const int64_t chunksB = grad_chunks(s.T, 0, s.N, s.r);
     w.partA = w.PtB + align256(2 * s.r * ldt * 2);
     w.partB = w.partA + align256(chunksA * s.r * s.K * 4);
     w.done = w.partB + align256(chunksB * s.r * s.N * 4);
@@ -274,10 +274,18 @@ int64_t bwd_total(const Shape& s) { return s.small ? sm_ws(s, false).total : bwd
 
 // The adapter rows on their own (the shrink's and the expand's adjoints), workspace layouts:
 // shrink: P [T, 2r] | Pt [2r, ldt] | At [K, r] | part [chunks, r, K] | done
-// expand: Bt [rd, N] | Pt2 [2r, ldt] | part [chunks, r, N] | done
+// expand: Bc [N, r] (B copied, when the caller's lies off 16 bytes) | Pt2 [2r, ldt] | part [chunks, r, N]
+// | done
+// With few tokens (few_adapter) the shrink needs none and the expand tpart [SD, T, r] f32; the sizes are
+// the larger of the two forms' (operands off their alignment take the other).
 struct ShrinkWs {
     int64_t P, Pt, At, part, done, total;
 };
+// Whether the adapter's adjoints on their own run as the few-token path's launches (f32 FMAs, the
+// partial sums few): measured, expand + shrink, at 32 tokens x 2048 columns x rank 16 23 us against 32, 256 x
+// 12288 x 16 30 against 53, 512 x 12288 x 16 57 against 58, 256 x 12288 x 64 102 against 111; past the
+// line 1024 x 2048 x 16 45 against 42, 512 x 12288 x 64 176 against 136.
+bool few_adapter(int64_t T, int r) { return T <= (r <= 16 ? 512 : 256); }
 ShrinkWs shrink_ws(int64_t T, int64_t K, int r) {
     ShrinkWs w{};
     if (r == 0) return w;
@@ -286,22 +294,24 @@ ShrinkWs shrink_ws(int64_t T, int64_t K, int r) {
     w.Pt = w.P + align256(T * 2 * r * 2);
     w.At = w.Pt + align256(2 * r * ldt * 2);
     w.part = w.At + align256(K * r * 2);
-    w.done = w.part + align256(grad_chunks(T, K, 0) * r * K * 4);
+    w.done = w.part + align256(grad_chunks(T, K, 0, r) * r * K * 4);
     w.total = w.done + align256(grad_blocks(K) * 4);
     return w;
 }
 struct ExpandWs {
-    int64_t Bt, Pt2, part, done, total;
+    int64_t Bc, Pt2, part, done, total;
 };
 ExpandWs expand_ws(int64_t T, int64_t N, int r) {
     ExpandWs w{};
     if (r == 0) return w;
     const int64_t ldt = grad_ld(T);
-    w.Bt = 0;
-    w.Pt2 = w.Bt + align256((int64_t)down_rank(r) * N * 2);
+    w.Bc = 0;
+    w.Pt2 = w.Bc + align256(N * r * 2);
     w.part = w.Pt2 + align256(2 * r * ldt * 2);
-    w.done = w.part + align256(grad_chunks(T, 0, N) * r * N * 4);
+    w.done = w.part + align256(grad_chunks(T, 0, N, r) * r * N * 4);
     w.total = w.done + align256(grad_blocks(N) * 4);
+    const int64_t few = few_adapter(T, r) ? align256((int64_t)sm_down_ranges(T, N) * T * r * 4) : 0;
+    if (few > w.total) w.total = few;
     return w;
 }
 
@@ -321,7 +331,7 @@ ShrinkQWs shrink_q_ws(int64_t T, int64_t K, int r) {
     w.xhi = w.g + align256(T * K * 4);
     w.xlo = w.xhi + align256(T * K * 2);
     w.part = w.xlo + align256(T * K * 2);
-    w.done = w.part + align256(grad_chunks(T, K, 0) * r * K * 4);
+    w.done = w.part + align256(grad_chunks(T, K, 0, r) * r * K * 4);
     w.total = w.done + align256(grad_blocks(K) * 4);
     return w;
 }
@@ -397,6 +407,7 @@ int sm_products(const R97qWeight* w, bool fwd, const Shape& sh, const uint16_t* 
     p.w.K = sh.K;
     p.act = act;
     p.F = F;
+    p.fvec = reinterpret_cast<uintptr_t>(F) % 16 == 0;
     p.rank = sh.r;
     p.S = ws.S;
     const int bm = sm::tile_tokens(sh.T);
@@ -446,6 +457,7 @@ void sm_output(sm::Finish& f, const Shape& sh, bool fwd, const uint16_t* F, void
     f.S = ws.S;
     f.outs = fwd ? sh.N : sh.K;
     f.F = F;
+    f.fvec = reinterpret_cast<uintptr_t>(F) % 8 == 0;
     f.out = out;
     f.out_f32 = dtype == R97Q_F32;
     f.accumulate = accumulate != 0;
@@ -665,7 +677,7 @@ int bwd_prep(const Shape& sh, const uint16_t* dY, const uint16_t* A, const uint1
 
 // the token chunks of the gradient launch for the factor gradients asked for
 int64_t grad_launch_chunks(const Shape& sh, bool dA, bool dB) {
-    const int64_t chunk = grad_chunk_rows(sh.T, dA ? sh.K : 0, dB ? sh.N : 0);
+    const int64_t chunk = grad_chunk_rows(sh.T, dA ? sh.K : 0, dB ? sh.N : 0, sh.r);
     return (grad_ld(sh.T) + chunk - 1) / chunk;
 }
 
@@ -677,7 +689,7 @@ int bwd_grads(const Shape& sh, const uint16_t* X, const uint16_t* dY, float* dA,
     GradArgs g{};
     g.T = sh.T;
     g.ldt = grad_ld(sh.T);
-    g.chunk = grad_chunk_rows(sh.T, dA ? sh.K : 0, dB ? sh.N : 0);
+    g.chunk = grad_chunk_rows(sh.T, dA ? sh.K : 0, dB ? sh.N : 0, sh.r);
     g.defer = defer;
     int nz = 0;
     int* done = reinterpret_cast<int*>(wsb + ws.done);
@@ -1038,12 +1050,13 @@ int r97q_lora_shrink_q_bwd(int64_t T, int64_t K, const void* a, int32_t a_dtype,
     uint16_t* P = reinterpret_cast<uint16_t*>(wsb + ws.P);
     uint16_t* Pt = reinterpret_cast<uint16_t*>(wsb + ws.Pt);
     int* done = reinterpret_cast<int*>(wsb + ws.done);
-    if (int e = launch_split(t_cot, T, rank, ldt, 1.0f, P, dA ? Pt : nullptr, done, (int)grad_blocks(K), s)) return e;
+    uint16_t* At = reinterpret_cast<uint16_t*>(wsb + ws.At);
+    if (int e = launch_split(t_cot, T, rank, ldt, 1.0f, P, dA ? Pt : nullptr, done, (int)grad_blocks(K), A,
+                             da || ds ? At : nullptr, K, s))
+        return e;
     if (da || ds) {
         // g = t_cot . A, then its two code-basis cotangents
-        uint16_t* At = reinterpret_cast<uint16_t*>(wsb + ws.At);
         float* g = reinterpret_cast<float*>(wsb + ws.g);
-        if (int e = launch_transpose2(nullptr, nullptr, 0, A, At, K, rank, s)) return e;
         if (int e = launch_lora_up(P, At, T, K, rank, g, 0, s)) return e;
         if (int e = launch_coded_cot(g, a, code_f32, a_scale, T, K, groups, gw, da, ds, s)) return e;
     }
@@ -1056,7 +1069,7 @@ int r97q_lora_shrink_q_bwd(int64_t T, int64_t K, const void* a, int32_t a_dtype,
             GradArgs g{};
             g.T = T;
             g.ldt = ldt;
-            g.chunk = grad_chunk_rows(T, K, 0);
+            g.chunk = grad_chunk_rows(T, K, 0, rank);
             g.one[0] = GradOne{Pt, x, K, dA, 1.0f, 0, reinterpret_cast<float*>(wsb + ws.part), done};
             if (int e = launch_lora_grads(rank, g, 1, s)) return e;
         }
@@ -1087,21 +1100,41 @@ int r97q_lora_shrink_bwd(int64_t T, int64_t K, const uint16_t* X, const uint16_t
     if (int e = check_ws(workspace_bytes, ws.total, workspace, who)) return e;
     uint8_t* wsb = static_cast<uint8_t*>(workspace);
     const hipStream_t s = (hipStream_t)stream;
+    if (few_adapter(T, rank)) {  // one launch: dX and dA from the f32 t_cot
+        sm::Finish f{};
+        f.T = T;
+        f.rank = rank;
+        f.U = t_cot;
+        f.SU = 1;
+        f.scale = 1.0f;
+        f.outs = K;
+        f.F = A;
+        f.fvec = reinterpret_cast<uintptr_t>(A) % 8 == 0;
+        f.out = dX;
+        f.out_f32 = 1;
+        f.accumulate = dx_accumulate != 0;
+        f.vec = reinterpret_cast<uintptr_t>(dX) % 16 == 0;
+        f.X = X;
+        f.K = K;
+        f.dA = dA;
+        return sm::launch_finish(f, s);
+    }
     const int64_t ldt = grad_ld(T);
     uint16_t* P = reinterpret_cast<uint16_t*>(wsb + ws.P);
     uint16_t* Pt = reinterpret_cast<uint16_t*>(wsb + ws.Pt);
     uint16_t* At = reinterpret_cast<uint16_t*>(wsb + ws.At);
     int* done = reinterpret_cast<int*>(wsb + ws.done);
-    if (int e = launch_split(t_cot, T, rank, ldt, 1.0f, P, dA ? Pt : nullptr, done, (int)grad_blocks(K), s)) return e;
+    if (int e = launch_split(t_cot, T, rank, ldt, 1.0f, P, dA ? Pt : nullptr, done, (int)grad_blocks(K), A,
+                             dX ? At : nullptr, K, s))
+        return e;
     if (dX) {
-        if (int e = launch_transpose2(nullptr, nullptr, 0, A, At, K, rank, s)) return e;
         if (int e = launch_lora_up(P, At, T, K, rank, dX, dx_accumulate, s)) return e;
     }
     if (dA) {
         GradArgs g{};
         g.T = T;
         g.ldt = ldt;
-        g.chunk = grad_chunk_rows(T, K, 0);
+        g.chunk = grad_chunk_rows(T, K, 0, rank);
         g.one[0] = GradOne{Pt, X, K, dA, 1.0f, 0, reinterpret_cast<float*>(wsb + ws.part), done};
         if (int e = launch_lora_grads(rank, g, 1, s)) return e;
     }
@@ -1131,13 +1164,50 @@ int r97q_lora_expand_bwd(int64_t T, int64_t N, const uint16_t* dY, const uint16_
     if (int e = check_ws(workspace_bytes, ws.total, workspace, who)) return e;
     uint8_t* wsb = static_cast<uint8_t*>(workspace);
     const hipStream_t s = (hipStream_t)stream;
+    if (few_adapter(T, rank) && reinterpret_cast<uintptr_t>(B) % 16 == 0) {
+        // two launches: dY.B over ranges, then t_cot and dB
+        sm::Finish f{};
+        f.T = T;
+        f.rank = rank;
+        f.U = static_cast<const float*>(workspace);
+        f.SU = sm_down_ranges(T, N);
+        f.scale = scale;
+        f.u_out = t_cot;
+        f.u_add = 1;
+        f.dY = dY;
+        f.t = t;
+        f.tscale = scale;
+        f.N = N;
+        f.dB = dB;
+        if (t_cot) {
+            sm::Params p{};
+            p.w.T = T;
+            p.w.N = N;
+            p.act = dY;
+            p.F = B;
+            p.rank = rank;
+            p.SD = f.SU;
+            p.mblocks = (int)((T + 31) / 32);
+            p.ndown = p.mblocks * p.SD;
+            p.tpart = static_cast<float*>(workspace);
+            sm::launch_products<R97Q_CODES8>(p, false, s);  // the down product alone reads no weight
+            if (int e = launch_status("sm_products_kernel")) return e;
+        }
+        return sm::launch_finish(f, s);
+    }
     const int64_t ldt = grad_ld(T);
-    uint16_t* Bt = reinterpret_cast<uint16_t*>(wsb + ws.Bt);
     uint16_t* Pt2 = reinterpret_cast<uint16_t*>(wsb + ws.Pt2);
-    if (int e = launch_transpose2(B, Bt, N, nullptr, nullptr, 0, rank, s)) return e;
+    if (reinterpret_cast<uintptr_t>(B) % 16 != 0) {  // the down product reads B in 16-byte pieces
+        uint16_t* Bc = reinterpret_cast<uint16_t*>(wsb + ws.Bc);
+        hipLaunchKernelGGL(pad_rows16, dim3((unsigned)((N * rank + 255) / 256)), dim3(256), 0, s, B, (int)N, (int)N,
+                           (int64_t)rank, Bc);
+        if (int e = launch_status("pad_rows16")) return e;
+        B = Bc;
+    }
     DownArgs a{};
     a.In = dY;
-    a.W = Bt;
+    a.W = B;
+    a.w_kmajor = 1;
     a.T = T;
     a.Kin = N;
     a.ldt = dB ? ldt : T;
@@ -1158,7 +1228,7 @@ int r97q_lora_expand_bwd(int64_t T, int64_t N, const uint16_t* dY, const uint16_
         GradArgs g{};
         g.T = T;
         g.ldt = ldt;
-        g.chunk = grad_chunk_rows(T, 0, N);
+        g.chunk = grad_chunk_rows(T, 0, N, rank);
         g.one[0] = GradOne{Pt2, dY, N, dB, 1.0f, 1, reinterpret_cast<float*>(wsb + ws.part),
                            reinterpret_cast<int*>(wsb + ws.done)};
         if (int e = launch_lora_grads(rank, g, 1, s)) return e;

@@ -24,6 +24,7 @@ struct Params {
     rt::Params w;         // the weight: stream, scale_t, a24, b, run_rows, N, K; and T
     const uint16_t* act;  // X [T, K] (forward) or dY [T, N] (dX), row-major
     const uint16_t* F;    // the down product's factor: A [r, K] (forward) or B [N, r] (dX)
+    int fvec;             // F takes 16-byte loads (A as the caller holds it may not: a value at a time)
     int rank;
     int S;                // ranges the products' reduction is dealt over
     int SD;               // and the down product's
@@ -46,17 +47,19 @@ struct Finish {
     int SU;
     float scale;
     // Y or dX [T, outs] (+)= sum over z < S of part[z] + u . F^T (forward: F = B [outs, r]) or
-    // u . F (dX: F = A [r, outs]); null part: none
+    // u . F (dX: F = A [r, outs]); S may be 0; null out: none
     const float* part;
     int S;
     int64_t outs;
     const uint16_t* F;
+    int fvec;  // F takes 16-byte (forward) or 8-byte (dX) loads
     int fwd;
     void* out;
     int out_f32, accumulate, vec;  // vec: out takes 4-value accesses
-    // t_out [T, r] = sum over z of U[z]; u_out [T, r] = u (either may be null)
+    // t_out [T, r] = sum over z of U[z]; u_out [T, r] = u (+= with u_add; either may be null)
     float* t_out;
     float* u_out;
+    int u_add;
     // dA [r, K] += u^T . X, dB [N, r] += tscale * dY^T . t (either may be null)
     const uint16_t* X;
     int64_t K;

@@ -391,7 +391,13 @@ __device__ __forceinline__ void down_item(const Params& p, uint8_t* lds, int mb,
                 const uint16_t* fp = p.F + (int64_t)(j < r ? j : 0) * n + (int64_t)s * kStep + 32 * half;
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    u32x4 v = *reinterpret_cast<const u32x4*>(fp + 8 * q);
+                    u32x4 v;
+                    if (p.fvec) {
+                        v = *reinterpret_cast<const u32x4*>(fp + 8 * q);
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) v[i] = (uint32_t)fp[8 * q + 2 * i] | (uint32_t)fp[8 * q + 2 * i + 1] << 16;
+                    }
                     if (j >= r) v = u32x4{0u, 0u, 0u, 0u};
                     f[q] = __builtin_bit_cast(bf16x8, v);
                 }

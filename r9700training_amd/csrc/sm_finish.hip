@@ -106,7 +106,11 @@ __device__ __forceinline__ void output_item(const Finish& f, float* u, int64_t m
         for (int j = 0; j < r; j += 8) {
             uint2 a[8];
 #pragma unroll
-            for (int q = 0; q < 8; ++q) a[q] = *reinterpret_cast<const uint2*>(f.F + (int64_t)(j + q) * f.outs + c);
+            for (int q = 0; q < 8; ++q) {
+                const uint16_t* p = f.F + (int64_t)(j + q) * f.outs + c;
+                a[q] = f.fvec ? *reinterpret_cast<const uint2*>(p)
+                              : uint2{(uint32_t)p[0] | (uint32_t)p[1] << 16, (uint32_t)p[2] | (uint32_t)p[3] << 16};
+            }
 #pragma unroll
             for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -261,7 +265,7 @@ __global__ __launch_bounds__(kThreads, R <= 32 ? 4 : 2) void sm_finish_kernel(co
             if (f.t_out || f.u_out) {
                 const float v = sum_ranges(f.U, f.SU, tr, i);
                 if (f.t_out) f.t_out[i] = v;
-                if (f.u_out) f.u_out[i] = f.scale * v;
+                if (f.u_out) f.u_out[i] = f.u_add ? f.u_out[i] + f.scale * v : f.scale * v;
             }
             if (f.ts) f.ts[i] = f.tscale * f.t[i];
             return;
@@ -278,7 +282,7 @@ __global__ __launch_bounds__(kThreads, R <= 32 ? 4 : 2) void sm_finish_kernel(co
 
 int launch_finish(const Finish& f, hipStream_t s) {
     Counts n{};
-    if (f.part) {
+    if (f.out) {
         n.ctiles = (int)(f.outs / kCols);
         n.outputs = (int)((f.T + kRows - 1) / kRows) * n.ctiles;
     }

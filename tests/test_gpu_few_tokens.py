@@ -135,3 +135,35 @@ def test_stages_keep_their_operands(T, N, K, r):
     assert torch.equal(Y, Ys) and torch.equal(dX, dXs) and torch.equal(Y, Yn)
     if r:
         assert torch.equal(t, ts) and torch.equal(dA, dAs) and torch.equal(dB, dBs) and torch.equal(t, tn)
+
+
+@pytest.mark.parametrize("T,C,r", [(1, 128, 8), (33, 640, 64), (256, 384, 64), (257, 384, 32), (512, 256, 16),
+                                   (513, 256, 16)])
+@pytest.mark.parametrize("off", [False, True])
+def test_adapter_adjoints(T, C, r, off):
+    """The adapter's adjoints on their own on both sides of the few-token line, the factors and dX in views
+    off their alignment too, against float64 products: f32 sums (few tokens) or two bf16 halves of the
+    f32 activations (16 bits) in bf16 products, 2e-5 relative."""
+    from r9700training_amd.qlinear import lora_expand_bwd, lora_shrink_bwd
+
+    print(f"case adapter adjoints T={T} C={C} r={r} off={off}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(T + r)
+
+    def rnd(shape, dtype=torch.float32):
+        n = shape[0] * shape[1]
+        v = torch.empty(n + 1, dtype=dtype, device="cuda")[int(off):][:n].view(shape)
+        return v.copy_(torch.randn(shape, generator=g, device="cuda"))
+
+    X = torch.randn((T, C), generator=g, device="cuda").to(torch.bfloat16)
+    A, B = rnd((r, C), torch.bfloat16), rnd((C, r), torch.bfloat16)
+    t, u, dX0 = rnd((T, r)), rnd((T, r)), rnd((T, C))
+    t_cot, dB = lora_expand_bwd(X, B, 2.0, t=t, t_cot=u.clone())
+    dX, dA = lora_shrink_bwd(X, A, t_cot, dX=rnd((T, C)).copy_(dX0), accumulate=True)
+    dX2, _ = lora_shrink_bwd(None, A, t_cot, want_dA=False)
+    torch.cuda.synchronize()
+    x, a, b = X.double(), A.double(), B.double()
+    want = u.double() + 2.0 * (x @ b)
+    tc = t_cot.double()
+    for got, ref in ((t_cot, want), (dB, 2.0 * (x.T @ t.double())), (dX, dX0.double() + tc @ a), (dX2, tc @ a),
+                     (dA, tc.T @ x)):
+        assert _rel(got, ref) <= 2e-5, _rel(got, ref)
