@@ -84,6 +84,16 @@ int launch_split(const float* U, int64_t T, int r, int64_t ldt, float scale, uin
 //   da or ds may be null)
 int launch_coded_cot(const float* g, const void* code, int code_f32, const float* a_scale, int64_t T, int64_t K,
                      int64_t groups, int64_t gw, float* da, float* ds, hipStream_t s);
+// da and ds of int8 codes from the up-projection's operands (launch_lora_up's P, Q), g never written; where
+// coded_up_takes
+bool coded_up_takes(int64_t gw, int64_t K, int64_t groups);
+int launch_coded_up(const uint16_t* P, const uint16_t* Q, const int8_t* code, const float* a_scale, int64_t T, int64_t K,
+                    int64_t groups, int64_t gw, int r, float* da, float* ds, hipStream_t s);
+// dA [r, K] += t^T . (code * scale): t f32 [T, r], int8 codes, where grads_coded_takes; part and done as a
+// GradOne's over K columns
+bool grads_coded_takes(int64_t gw, int64_t K, int64_t groups);
+int launch_grads_coded(int r, const float* t, const int8_t* code, const float* scale, int64_t T, int64_t K,
+                       int64_t groups, int64_t gw, float* dA, float* part, int* done, hipStream_t s);
 //   x = code * a_scale as [hi | lo] bf16 [T, K] each
 int launch_coded_x(const void* code, int code_f32, const float* a_scale, int64_t T, int64_t K, int64_t groups,
                    int64_t gw, uint16_t* xhi, uint16_t* xlo, hipStream_t s);

@@ -1054,12 +1054,21 @@ int r97q_lora_shrink_q_bwd(int64_t T, int64_t K, const void* a, int32_t a_dtype,
     if (int e = launch_split(t_cot, T, rank, ldt, 1.0f, P, dA ? Pt : nullptr, done, (int)grad_blocks(K), A,
                              da || ds ? At : nullptr, K, s))
         return e;
-    if (da || ds) {
+    // int8 codes from 16-byte-aligned rows with groups that fit the kernels' 64-column waves: one launch for
+    // the two cotangents, one for dA; the others through the values g and x
+    const int8_t* codes = code_f32 || reinterpret_cast<uintptr_t>(a) % 16 != 0 ? nullptr : static_cast<const int8_t*>(a);
+    const bool up = codes && coded_up_takes(gw, K, groups), grads = codes && grads_coded_takes(gw, K, groups);
+    if ((da || ds) && up) {
+        if (int e = launch_coded_up(P, At, codes, a_scale, T, K, groups, gw, rank, da, ds, s)) return e;
+    } else if (da || ds) {
         // g = t_cot . A, then its two code-basis cotangents
         float* g = reinterpret_cast<float*>(wsb + ws.g);
         if (int e = launch_lora_up(P, At, T, K, rank, g, 0, s)) return e;
         if (int e = launch_coded_cot(g, a, code_f32, a_scale, T, K, groups, gw, da, ds, s)) return e;
     }
+    if (dA && grads)
+        return launch_grads_coded(rank, t_cot, codes, a_scale, T, K, groups, gw, dA, reinterpret_cast<float*>(wsb + ws.part),
+                                  done, s);
     if (dA) {
         // dA += t_cot^T . x with x = [hi | lo](a * a_scale): two gradient passes, one a half
         uint16_t* xhi = reinterpret_cast<uint16_t*>(wsb + ws.xhi);

@@ -228,3 +228,31 @@ def test_coded_entry_refusals():
         lora_shrink_q_bwd(torch.zeros((8, 256), dtype=torch.int8, device="cuda"),
                           torch.ones((8, 3), device="cuda"), torch.zeros((16, 256), dtype=torch.bfloat16, device="cuda"),
                           torch.zeros((8, 16), device="cuda"), group_width=128)
+
+
+@pytest.mark.parametrize("T,K,gw,r", [(5, 128, 64, 8), (33, 384, 128, 16), (200, 768, 256, 64), (70, 1152, 128, 32),
+                                      (129, 1024, 512, 16), (64, 896, 96, 16), (1, 640, 128, 64), (700, 256, 64, 64)])
+def test_int8_codes_match_the_general_path(T, K, gw, r):
+    """The coded shrink's adjoint over int8 codes with group widths the fused kernels take (64, 128, 256
+    columns; a multiple of 256 for dA) and others, against the same codes handed over as f32 values,
+    which take the general path: the two hold the f32 operands as two bf16 halves each (16 bits), the
+    general one the activation's value, the fused one the scaled cotangent -- 2e-5 relative."""
+    from r9700training_amd.qlinear import lora_shrink_q_bwd
+
+    print(f"case coded shrink T={T} K={K} gw={gw} r={r}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(T + K)
+    groups = (K + gw - 1) // gw
+    code = torch.randint(-128, 128, (T, K), generator=g, device="cuda", dtype=torch.int8)
+    s = 0.01 + torch.rand((T, groups), generator=g, device="cuda")
+    A = (0.1 * torch.randn((r, K), generator=g, device="cuda")).to(torch.bfloat16)
+    t = torch.randn((T, r), generator=g, device="cuda")
+    base = [torch.randn(sh, generator=g, device="cuda") for sh in ((T, K), (T, groups), (r, K))]
+    out = [lora_shrink_q_bwd(a, s, A, t, da=base[0].clone(), ds=base[1].clone(), dA=base[2].clone(), group_width=gw)
+           for a in (code, code.float(), code)]
+    only = lora_shrink_q_bwd(code, s, A, t, ds=base[1].clone(), want=("ds",), group_width=gw)
+    torch.cuda.synchronize()
+    for i, (a, b, c) in enumerate(zip(*out)):
+        assert torch.equal(a, c), i
+        d = (b - base[i]).double()
+        assert float((a.double() - b.double()).norm() / d.norm()) <= 2e-5, i
+    assert torch.equal(only[1], out[0][1])
