@@ -725,6 +725,34 @@ int dx_base(const R97qWeight* w, const Shape& sh, void* dX, int32_t dx_dtype, in
 // epilogue (no adapter, no workspace)
 int dx_scaled(const R97qWeight* w, const Shape& sh, const uint16_t* dY, void* dX, int32_t dx_dtype,
               int32_t accumulate, hipStream_t s, const float* a_scale) {
+    if (const int bm = sm::coded_tile(sh.T, sh.K)) {
+        sm::Params p{};
+        p.w.T = sh.T;
+        p.w.N = sh.N;
+        p.w.K = sh.K;
+        p.w.stream = w->stream;
+        p.w.scale_t = w->scale_t;
+        p.w.a24 = w->mad_a & 0xFFFFFFu;
+        p.w.b = w->mad_b;
+        p.w.run_rows = w->run_rows;
+        p.w.out = dX;
+        p.w.out_f32 = dx_dtype == R97Q_F32;
+        p.w.accumulate = accumulate != 0;
+        p.act = dY;
+        p.S = 1;
+        p.mtiles = (int)((sh.T + bm - 1) / bm);
+        p.otiles = (int)(sh.K / kBN);
+        p.nprod = p.mtiles * p.otiles;
+        p.a_scale = a_scale;
+        switch (w->bits) {
+            case 3: sm::launch_coded_dx<3>(p, bm, s); break;
+            case 4: sm::launch_coded_dx<4>(p, bm, s); break;
+            case 5: sm::launch_coded_dx<5>(p, bm, s); break;
+            case 6: sm::launch_coded_dx<6>(p, bm, s); break;
+            default: sm::launch_coded_dx<R97Q_CODES8>(p, bm, s); break;
+        }
+        return launch_status("sm_coded_dx_kernel");
+    }
     DxParams p{};
     p.a_scale = a_scale;
     p.a_scale_ld = sh.K / kBN;

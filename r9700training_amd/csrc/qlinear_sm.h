@@ -34,9 +34,23 @@ struct Params {
     int nprod;            // product workgroups: mtiles * otiles * S, or 0
     float* part;          // [S][T][outputs]
     float* tpart;         // [SD][T][r]
+    const float* a_scale; // launch_coded_dx: f32 [T, otiles]
 };
 template <int BITS>
 void launch_products(const Params& p, bool fwd, hipStream_t s);
+
+// gemm_nt_q's adjoint (w.out (+)= a_scale[m, k/128] * (act . W)[m, k]; S 1, nprod tiles) with tiles of
+// `tile` tokens, and the tile it takes: the smallest of 32 (up to 32 tokens), 64 (up to 64), 128 and 256
+// with at most a tile a CU, or 0 where 256 are still more (the 512-token tiles then fill the chip)
+template <int BITS>
+void launch_coded_dx(const Params& p, int tile, hipStream_t s);
+inline int coded_tile(int64_t T, int64_t K) {
+    if (T <= 32) return 32;
+    if (T <= 64) return 64;
+    for (int bm : {128, 256})
+        if ((T + bm - 1) / bm * (K / 128) <= 256) return bm;
+    return 0;
+}
 
 // One finishing launch: the parts whose counts are non-zero. `u` below is scale * sum over z < SU of
 // U[z] (f32 [T, r] each): s.t in the forward, dt in the backward.

@@ -251,22 +251,24 @@ __device__ __forceinline__ void load_tokens(const uint16_t* row, int s, uint4 (&
     for (int j = 0; j < NJ; ++j) t[j] = *reinterpret_cast<const uint4*>(row + (int64_t)s * kStep + 8 * j);
 }
 
-// A product workgroup: MT token blocks of 32. With four, a wave takes one block and two of the four
-// 32-output blocks; with two, one block and one output block; with one, one output block and half of
+// A product workgroup: MT token blocks of 32. With eight, a wave takes one block and all four 32-output
+// blocks; with four, one block and two output blocks; with two, one block and one output block; with one, one output block and half of
 // each step's reduction (two of its four 16-deep slices), the halves added at the end. A step's
 // tokens are read whole-row (eight lanes a 128-byte line) and go through LDS in the weight tile's
 // layout: as fragments straight from the rows, 32 lines an instruction and every block loaded by as many
 // waves as share it, the loads cost more than the decode.
-template <bool FWD, int MT>
+// DIRECT: the whole reduction (S 1), the product in the code basis of an activation written (or added)
+// into the output: times a_scale[m, output tile]; else the range's partial.
+template <bool FWD, int MT, bool DIRECT = false>
 __device__ __forceinline__ void product_item(const Params& p, uint8_t* tiles, uint8_t* toks, int mt, int ot, int z) {
-    constexpr int NN = MT == 4 ? 2 : 1;
+    constexpr int NN = MT == 8 ? 4 : MT == 4 ? 2 : 1;
     constexpr int NJ = MT == 1 ? 2 : 4;
-    constexpr int NT = MT == 4 ? 2 : 1;  // 16-byte token pieces a thread loads a step
+    constexpr int NT = MT >= 4 ? MT / 2 : 1;  // 16-byte token pieces a thread loads a step
     constexpr int kTokBytes = MT * 32 * 2 * kStep;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int half = lane >> 5, l32 = lane & 31;
-    const int blk = MT == 4 ? wave >> 1 : MT == 2 ? wave >> 2 : 0;
-    const int ni0 = MT == 4 ? 2 * (wave & 1) : wave & 3;
+    const int blk = MT == 8 ? wave : MT == 4 ? wave >> 1 : MT == 2 ? wave >> 2 : 0;
+    const int ni0 = MT == 8 ? 0 : MT == 4 ? 2 * (wave & 1) : wave & 3;
     const int j0 = MT == 1 ? 2 * (wave >> 2) : 0;
     const int64_t red = FWD ? p.w.K : p.w.N, outs = FWD ? p.w.N : p.w.K;
     int s0, s1;
@@ -347,6 +349,28 @@ __device__ __forceinline__ void product_item(const Params& p, uint8_t* tiles, ui
         for (int e = 0; e < 16; ++e) acc[0][e] += h[64 * e + lane];
     }
     // accumulator element e: row 8*(e/4) + 4*half + e%4 of the block, column 32 ni + l32
+    if constexpr (DIRECT) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int64_t m = m0 + 8 * (e >> 2) + 4 * half + (e & 3);
+            if (m >= p.w.T) continue;
+            const float f = p.a_scale[m * p.otiles + ot];
+            const int64_t at = m * outs + o0 + 32 * ni0 + l32;
+#pragma unroll
+            for (int ni = 0; ni < NN; ++ni) {
+                float v = acc[ni][e] * f;
+                if (p.w.out_f32) {
+                    float* d = static_cast<float*>(p.w.out) + at + 32 * ni;
+                    *d = p.w.accumulate ? *d + v : v;
+                } else {
+                    uint16_t* d = static_cast<uint16_t*>(p.w.out) + at + 32 * ni;
+                    if (p.w.accumulate) v += bf16_to_f32(*d);
+                    *d = f32_to_bf16(v);
+                }
+            }
+        }
+        return;
+    }
     float* out = p.part + (int64_t)z * p.w.T * outs + o0 + 32 * ni0 + l32;
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
@@ -461,7 +485,30 @@ __global__ __launch_bounds__(64 * kWaves, 4) void sm_products_kernel(const Param
     product_item<FWD, MT>(p, tiles, toks, mt, q % p.otiles, q / p.otiles);
 }
 
+// gemm_nt_q's adjoint where the 512-token tiles of qlinear_fused.hip would leave CUs idle: the whole
+// reduction a workgroup, as many token blocks a tile as keep the tiles within one a CU (sm::coded_tile).
+// Measured at 4096 x 4096, int8-code weight, with the call's gap: 1 token 30 us, 128 tokens 46, 1024
+// tokens 57, 2048 tokens 90, against 98, 105, 120 and 127.
+template <int MT>
+__global__ __launch_bounds__(64 * kWaves, MT == 8 ? 2 : 4) void sm_coded_dx_kernel(const Params p) {
+    __shared__ __attribute__((aligned(16))) uint8_t tiles[2 * kTileBytes];
+    __shared__ __attribute__((aligned(16))) uint8_t toks[2 * MT * 32 * 2 * kStep];
+    const int i = rt::xcd_tile(blockIdx.x, p.nprod);
+    product_item<false, MT, true>(p, tiles, toks, i % p.mtiles, i / p.mtiles, 0);
+}
+
 }  // namespace
+
+template <>
+void launch_coded_dx<R97Q_BITS>(const Params& p, int tile, hipStream_t s) {
+    const dim3 grid((unsigned)p.nprod), block(64 * kWaves);
+    switch (tile) {
+        case 32: hipLaunchKernelGGL(sm_coded_dx_kernel<1>, grid, block, 0, s, p); break;
+        case 64: hipLaunchKernelGGL(sm_coded_dx_kernel<2>, grid, block, 0, s, p); break;
+        case 128: hipLaunchKernelGGL(sm_coded_dx_kernel<4>, grid, block, 0, s, p); break;
+        default: hipLaunchKernelGGL(sm_coded_dx_kernel<8>, grid, block, 0, s, p); break;
+    }
+}
 
 template <>
 void launch_products<R97Q_BITS>(const Params& p, bool fwd, hipStream_t s) {

@@ -256,3 +256,67 @@ def test_int8_codes_match_the_general_path(T, K, gw, r):
         d = (b - base[i]).double()
         assert float((a.double() - b.double()).norm() / d.norm()) <= 2e-5, i
     assert torch.equal(only[1], out[0][1])
+
+
+@pytest.mark.parametrize("T,N,K,bf16", [(1, 128, 128, False), (31, 256, 640, True), (33, 384, 1152, False),
+                                        (100, 8192, 128, False), (130, 6528, 256, False), (129, 128, 4224, False)])
+def test_coded_forward_few_tokens(T, N, K, bf16):
+    """The coded forward on both sides of its few-token line (1024 tiles of 32 x 32: 100 x 8192 the last
+    of it, 130 x 6528 and beyond the larger tile) and off 16 bytes, against float64: the group sums are
+    exact, so what is left is the f32 fold over the groups (1e-6 relative) and a bf16 output's rounding."""
+    from r9700training_amd.qlinear import gemm_nt_q_fwd
+
+    print(f"case coded forward T={T} N={N} K={K} bf16={bf16}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(T * N + K)
+
+    def codes(rows):
+        return torch.randint(-127, 128, (rows, K), generator=g, device="cuda", dtype=torch.int8)
+
+    w, a = codes(N), codes(T)
+    ws = (0.001 + 0.01 * torch.rand((N, K // 128), generator=g, device="cuda")).to(torch.bfloat16)
+    s = 0.01 + torch.rand((T, K // 128), generator=g, device="cuda")
+    off = torch.empty(T * K + 1, dtype=torch.int8, device="cuda")[1:].view(T, K).copy_(a)
+    wide = lambda c, x: c.double() * x.double().repeat_interleave(128, 1)  # noqa: E731
+    ref = wide(a, s) @ wide(w, ws).T
+    dt = torch.bfloat16 if bf16 else torch.float32
+    for x in (a, off):
+        Y = gemm_nt_q_fwd(w, ws, x, s, y_dtype=dt)
+        torch.cuda.synchronize()
+        assert float((Y.double() - ref).norm() / ref.norm()) <= (2.5e-3 if bf16 else 1e-6)
+
+
+@pytest.mark.parametrize("T,N,K,bits", [(1, 128, 128, 5), (32, 384, 256, 3), (33, 256, 512, 8), (64, 640, 384, 4),
+                                        (65, 256, 1024, 6), (257, 128, 16384, 5), (513, 256, 16384, 8),
+                                        (1200, 128, 8192, 5)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_coded_dx_tiles(T, N, K, bits, dtype):
+    """gemm_nt_q's adjoint over its token tiles (32, 64, 128, 256 and 512 tokens), written and added to,
+    against the plain dX product's f32 output times the scale: the same bf16 products, so the order of
+    the f32 sums (1e-6) and a bf16 output's roundings are all that differ."""
+    from r9700training_amd import R97Q_DECODE_AUTO, R97Q_DECODE_FUSED, lib
+    from r9700training_amd.qlinear import QWeight, gemm_nt_q_dx, qlinear_lora_bwd
+    from gpu_util import device_desc
+
+    print(f"case coded dX T={T} N={N} K={K} bits={bits} {dtype}", flush=True)
+    keep = []
+    p = S.trellis(rows=N, cols=K, bits=5 if bits == 8 else bits, run_rows=128, rowf=True, seed=T, packed=True,
+                  scale_col=np.ones(K // 128, np.float32))
+    sc = torch.ones(K // 128, device="cuda")
+    w = QWeight(device_desc(p, keep), scale_col=sc, codes8=bits == 8)
+    g = torch.Generator(device="cuda").manual_seed(T + N)
+    dY = torch.randn((T, N), generator=g, device="cuda").to(torch.bfloat16)
+    s = 0.01 + torch.rand((T, K // 128), generator=g, device="cuda")
+    lib().r97q_set_decode_once(R97Q_DECODE_FUSED)
+    try:
+        plain, _, _ = qlinear_lora_bwd(w, None, dY, dx_dtype=torch.float32)
+    finally:
+        lib().r97q_set_decode_once(R97Q_DECODE_AUTO)
+    want = plain.double() * s.double().repeat_interleave(128, 1)
+    base = torch.randn((T, K), generator=g, device="cuda").to(dtype)
+    got = gemm_nt_q_dx(w, dY, s, da_dtype=dtype)
+    added = gemm_nt_q_dx(w, dY, s, dA=base.clone(), accumulate=True)
+    torch.cuda.synchronize()
+    tol = 1e-6 if dtype == torch.float32 else 2.5e-3
+    assert float((got.double() - want).norm() / want.norm()) <= tol
+    both = want + base.double()
+    assert float((added.double() - both).norm() / both.norm()) <= tol
