@@ -226,13 +226,13 @@ BwdWs bwd_ws(const Shape& s) {
 }
 
 // ---------------------------------------------------------------- the few-token path's layouts
-// The ranges the reduction of a product over T tokens is dealt over: about one workgroup a CU with
-// tiles of 32 and 64 tokens, two with 128 (measured at 4096 x 4096, forward + backward: at 32 tokens 256
-// workgroups 39 us, 512 46, 1024 69; at 128 tokens 65, 61, 89), two steps a range at least, and the
-// partials within kSmPartBytes
+// The ranges the reduction of a product over T tokens is dealt over: about one workgroup a CU, two at 65
+// to 128 tokens (measured, forward + backward: 32 x 4096 x 4096 with 256 workgroups 39 us, 512 46, 1024 69;
+// 128 x 4096 x 4096 65, 61, 89; 1024 x 1024 x 1024, where the partials are the cost, 70 with 256, 92 with
+// 512), two steps a range at least, and the partials within kSmPartBytes
 int sm_ranges(int64_t T, int64_t outputs, int64_t red) {
     const int64_t bm = sm::tile_tokens(T), tiles = (T + bm - 1) / bm * (outputs / kBN);
-    int64_t S = ((bm < 128 ? 256 : 512) + tiles - 1) / tiles;
+    int64_t S = ((T > 64 && T <= 128 ? 512 : 256) + tiles - 1) / tiles;
     const int64_t most = red / rt::kStep / 2, fit = kSmPartBytes / (T * outputs * 4);
     S = S < most ? S : most;
     S = S < fit ? S : fit;
