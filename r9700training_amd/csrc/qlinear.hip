@@ -505,6 +505,17 @@ int sm_bwd(const R97qWeight* w, const Shape& sh, const uint16_t* X, const uint16
     f.tscale = scale;
     f.N = sh.N;
     f.dB = dB;
+    // dX written over dY or X (as the path for more tokens allows): the gradients read them first
+    const auto over = [&](const void* in, int64_t bytes) {
+        const uintptr_t a = reinterpret_cast<uintptr_t>(dX), b = reinterpret_cast<uintptr_t>(in);
+        return in && a < b + bytes && b < a + sh.T * sh.K * (f.out_f32 ? 4 : 2);
+    };
+    if ((dA && over(X, sh.T * sh.K * 2)) || (dB && over(dY, sh.T * sh.N * 2))) {
+        f.out = nullptr;
+        if (int e = sm::launch_finish(f, s)) return e;
+        f.out = dX;
+        f.dA = f.dB = nullptr;
+    }
     return sm::launch_finish(f, s);
 }
 int sm_bwd_prep(const Shape& sh, const uint16_t* dY, const uint16_t* A, const uint16_t* B, const float* t, float scale,

@@ -97,6 +97,31 @@ def test_few_tokens_match_the_other_path(modes, T, N, K, r, bits, run, codes8, b
         assert torch.isfinite(a).all() and e <= (2 ** -8 if bf16 and i < 2 else 2e-5), (i, e)
 
 
+@pytest.mark.parametrize("over", ["X", "dY"])
+@pytest.mark.parametrize("T,r", [(5, 8), (130, 16), (300, 64)])
+def test_outputs_over_their_inputs(T, r, over):
+    """A bf16 Y written over X and a bf16 dX over X or dY (a square layer): the separate buffers' bits,
+    the factor gradients included, as on the path for more tokens."""
+    from r9700training_amd.qlinear import qlinear_lora_bwd, qlinear_lora_fwd
+
+    print(f"case few tokens in place T={T} r={r} over={over}", flush=True)
+    rng = np.random.default_rng(T)
+    keep = []
+    N = K = 512
+    w = _weight(N, K, 5, 128, False, T, keep)
+    X, dY = bf16_tensor(rng.standard_normal((T, K))), bf16_tensor(rng.standard_normal((T, N)))
+    A, B = bf16_tensor(0.01 * rng.standard_normal((r, K))), bf16_tensor(0.01 * rng.standard_normal((N, r)))
+    Y, t = qlinear_lora_fwd(w, X, A, B, 2.0, y_dtype=torch.bfloat16)
+    want = (Y, *qlinear_lora_bwd(w, X, dY, A, B, t, 2.0, dx_dtype=torch.bfloat16))
+    y = X.clone()
+    qlinear_lora_fwd(w, y, A, B, 2.0, out=y)
+    x, g = X.clone(), dY.clone()
+    dX, dA, dB = qlinear_lora_bwd(w, x, g, A, B, t, 2.0, dX=x if over == "X" else g)
+    torch.cuda.synchronize()
+    for a, b in zip((y, dX, dA, dB), want):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("T,N,K,r", [(7, 384, 512, 16), (130, 256, 384, 0), (300, 512, 256, 64)])
 def test_stages_keep_their_operands(T, N, K, r):
     """The stage entries on this path: the fused entries' bits, with X and dY overwritten between the
