@@ -24,8 +24,7 @@ namespace {
 constexpr int kThreads = 512;
 constexpr int kRows = 32;       // token rows of an output workgroup
 constexpr int kCols = 128;      // its columns: four a thread, two rows
-constexpr int kGradCols = 32;   // columns of a gradient workgroup: a lane a column, two rows a wave
-constexpr int kGradRows = 16;   // token rows a wave stages at a time
+constexpr int kGradCols = 32;   // columns of a gradient workgroup
 constexpr int kCopy = 32 * kThreads;  // values of a copy workgroup
 
 __device__ __forceinline__ float4 add4(float4 a, float4 b) { return {a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w}; }
@@ -157,78 +156,91 @@ __device__ __forceinline__ void output_item(const Finish& f, float* u, int64_t m
 }
 
 // out[j][c] or out[c][j] += sum over m of g[m][j] V[m][c] for the 32 columns from c0, g = mul * sum over
-// z < SU of U[z]. Wave w takes an eighth of the token rows, its lanes' upper half the odd ones; the
-// 16 sums of a column meet in LDS, added in order.
+// z < SU of U[z]. Wave w takes an eighth of the token rows; the eight sums of a column meet in LDS,
+// added in order. The products run on the f32 MFMAs (32 x 32 x 2; 16 x 16 x 4 up to rank 16, rank 8 with
+// zero rows): exact f32 operands and f32 sums as FMAs give, and a lane's operand is the value it loaded.
+// FMAs with g broadcast from LDS were bound by the LDS reads (16 bytes for four FMAs of a wave): the
+// 777-token, 2560 + 1408-column launch at rank 32 took 41 us, now 26.
 template <int R>
 __device__ __forceinline__ void grad_item(const float* U, int SU, float mul, int64_t T, const uint16_t* V, int64_t C, int64_t c0,
                           float* out, bool transposed, float* lds) {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, half = lane >> 5, l32 = lane & 31;
+    using Acc = float __attribute__((ext_vector_type(R >= 32 ? 16 : 4)));
     constexpr int kW = kThreads / 64;
-    const int64_t per = ((T + kW - 1) / kW + 1) & ~int64_t(1);
+    constexpr int kM = R >= 32 ? 32 : 16;     // an MFMA's factor rows and columns
+    constexpr int kRowsMf = 64 / kM;          // its token rows: lane / kM
+    constexpr int kJ = R > kM ? R / kM : 1;   // factor-row tiles
+    constexpr int kC = kGradCols / kM;        // column tiles
+    constexpr int kBatch = 16;  // token rows loaded at a time, the next while these multiply (32: no faster, and slower to 256 tokens)
+    constexpr int kN = kBatch / kRowsMf;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, hi = lane / kM, lo = lane % kM;
+    const int64_t per = ((T + kW - 1) / kW + kRowsMf - 1) / kRowsMf * kRowsMf;
     const int64_t b = wave * per, e = b + per < T ? b + per : T;
-    float* g = lds + wave * kGradRows * R;  // the wave's staged rows
-    float acc[R];
-#pragma unroll
-    for (int j = 0; j < R; ++j) acc[j] = 0.0f;
-    constexpr int kHold = kGradRows * R / 64;  // staged values a lane holds
-    float x[kGradRows / 2], h[kHold];
-    const int c32 = (int)C;
+    Acc acc[kJ][kC] = {};
+    float x[kN][kC], h[kN][kJ];
+    const int c32 = (int)C, lu = lo < R ? lo : 0;
+    // rows past e (and factor rows past R) load a valid element and count as zero
     auto load = [&](int64_t m) {
-        const uint16_t* vp = V + m * C + c0 + l32;
         const int rows = (int)(e - m);
+        const uint16_t* vp = V + m * C + c0 + lo;
 #pragma unroll
-        for (int i = 0; i < kGradRows / 2; ++i) {
-            const int row = 2 * i + half;
-            const uint16_t v = vp[row < rows ? row * c32 : 0];
-            x[i] = row < rows ? bf16_to_f32(v) : 0.0f;
+        for (int i = 0; i < kN; ++i) {
+            const int row = kRowsMf * i + hi;
+#pragma unroll
+            for (int c = 0; c < kC; ++c) {
+                const uint16_t v = vp[(row < rows ? row * c32 : 0) + c * kM];
+                x[i][c] = row < rows ? bf16_to_f32(v) : 0.0f;
+            }
         }
-        // rows past e read the last row's values (x is zero there)
-        const float* u = U + m * R + lane;
-        const int left = (int)(e - m) * R - 1 - lane;
+        const float* u = U + m * R + lu;
 #pragma unroll
-        for (int i = 0; i < kHold; ++i) h[i] = u[64 * i <= left ? 64 * i : left];
+        for (int i = 0; i < kN; ++i)
+#pragma unroll
+            for (int j = 0; j < kJ; ++j) h[i][j] = u[(kRowsMf * i + hi < rows ? kRowsMf * i + hi : 0) * R + j * kM];
         for (int z = 1; z < SU; ++z) {
             u += T * R;
 #pragma unroll
-            for (int i = 0; i < kHold; ++i) h[i] += u[64 * i <= left ? 64 * i : left];
+            for (int i = 0; i < kN; ++i)
+#pragma unroll
+                for (int j = 0; j < kJ; ++j) h[i][j] += u[(kRowsMf * i + hi < rows ? kRowsMf * i + hi : 0) * R + j * kM];
         }
 #pragma unroll
-        for (int i = 0; i < kHold; ++i) h[i] *= mul;
+        for (int i = 0; i < kN; ++i)
+#pragma unroll
+            for (int j = 0; j < kJ; ++j) h[i][j] = kRowsMf * i + hi < rows && lo < R ? mul * h[i][j] : 0.0f;
     };
     if (b < e) load(b);
-    for (int64_t m = b; m < e; m += kGradRows) {
-        // one wave's LDS operations run in order: the reads below see these writes, and the next rows'
-        // writes come after them
+    for (int64_t m = b; m < e; m += kBatch) {
+        float xc[kN][kC], hc[kN][kJ];
 #pragma unroll
-        for (int i = 0; i < kHold; ++i) g[lane + 64 * i] = h[i];
-        float xc[kGradRows / 2];
+        for (int i = 0; i < kN; ++i) {
 #pragma unroll
-        for (int i = 0; i < kGradRows / 2; ++i) xc[i] = x[i];
-        __builtin_amdgcn_wave_barrier();
-        if (m + kGradRows < e) load(m + kGradRows);  // on their way while these rows multiply
+            for (int c = 0; c < kC; ++c) xc[i][c] = x[i][c];
 #pragma unroll
-        for (int i = 0; i < kGradRows / 2; ++i) {
-            const float4* gr = reinterpret_cast<const float4*>(g + (2 * i + half) * R);
-#pragma unroll
-            for (int j = 0; j < R / 4; ++j) {
-                const float4 w = gr[j];
-                acc[4 * j] = __builtin_fmaf(w.x, xc[i], acc[4 * j]);
-                acc[4 * j + 1] = __builtin_fmaf(w.y, xc[i], acc[4 * j + 1]);
-                acc[4 * j + 2] = __builtin_fmaf(w.z, xc[i], acc[4 * j + 2]);
-                acc[4 * j + 3] = __builtin_fmaf(w.w, xc[i], acc[4 * j + 3]);
-            }
-            __builtin_amdgcn_sched_barrier(0);  // a row's reads at a time: registers
+            for (int j = 0; j < kJ; ++j) hc[i][j] = h[i][j];
         }
-        __builtin_amdgcn_wave_barrier();
-    }
+        if (m + kBatch < e) load(m + kBatch);  // on their way while these rows multiply
 #pragma unroll
-    for (int j = 0; j < R; ++j) acc[j] += __shfl_xor(acc[j], 32);
-    __syncthreads();
-    // [wave][R][32 columns]
-    if (half == 0) {
+        for (int i = 0; i < kN; ++i)
 #pragma unroll
-        for (int j = 0; j < R; ++j) lds[(wave * R + j) * kGradCols + l32] = acc[j];
+            for (int j = 0; j < kJ; ++j)
+#pragma unroll
+                for (int c = 0; c < kC; ++c) {
+                    if constexpr (kM == 32)
+                        acc[j][c] = __builtin_amdgcn_mfma_f32_32x32x2f32(hc[i][j], xc[i][c], acc[j][c], 0, 0, 0);
+                    else
+                        acc[j][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(hc[i][j], xc[i][c], acc[j][c], 0, 0, 0);
+                }
     }
+    // [wave][R][32 columns]; a lane holds factor rows 4 * (lane / kM) + .. of the column lane % kM
+#pragma unroll
+    for (int j = 0; j < kJ; ++j)
+#pragma unroll
+        for (int c = 0; c < kC; ++c)
+#pragma unroll
+            for (int q = 0; q < (kM == 32 ? 16 : 4); ++q) {
+                const int row = j * kM + q / 4 * 8 + 4 * hi + q % 4;
+                if (row < R) lds[(wave * R + row) * kGradCols + c * kM + lo] = acc[j][c][q];
+            }
     __syncthreads();
     for (int i = threadIdx.x; i < R * kGradCols; i += kThreads) {
         // neighbouring threads neighbouring elements of the output
@@ -241,17 +253,15 @@ __device__ __forceinline__ void grad_item(const float* U, int SU, float mul, int
 }
 
 struct Counts {
-    int outputs, dA, dB, rows, copies[2];  // workgroups of each kind, in this order
+    int dA, dB, outputs, rows, copies[2];  // workgroups of each kind, in this order (the longest first)
     int ctiles;
 };
 
 template <int R>
 __global__ __launch_bounds__(kThreads, R <= 32 ? 4 : 2) void sm_finish_kernel(const Finish f, const Counts n) {
-    // the gradients' sums [8][R][32]; the output's u [32][R]; the staged rows [8][16][R]
+    // the gradients' sums [8][R][32]; the output's u [32][R]
     __shared__ __attribute__((aligned(16))) float lds[8 * kGradCols * (R < 8 ? 8 : R)];
     int b = blockIdx.x;
-    if (b < n.outputs) return output_item(f, lds, (int64_t)(b / n.ctiles) * kRows, (int64_t)(b % n.ctiles) * kCols);
-    b -= n.outputs;
     if constexpr (R > 0) {
         if (b < n.dA + n.dB) {  // one call, so that it inlines
             const bool a = b < n.dA;
@@ -259,6 +269,10 @@ __global__ __launch_bounds__(kThreads, R <= 32 ? 4 : 2) void sm_finish_kernel(co
                                 (int64_t)(a ? b : b - n.dA) * kGradCols, a ? f.dA : f.dB, !a, lds);
         }
         b -= n.dA + n.dB;
+    }
+    if (b < n.outputs) return output_item(f, lds, (int64_t)(b / n.ctiles) * kRows, (int64_t)(b % n.ctiles) * kCols);
+    b -= n.outputs;
+    if constexpr (R > 0) {
         if (b < n.rows) {
             const int64_t i = (int64_t)b * kThreads + threadIdx.x, tr = f.T * R;
             if (i >= tr) return;
