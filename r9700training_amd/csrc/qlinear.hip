@@ -66,23 +66,27 @@ constexpr int64_t kDecodeOnceMinTLarge = 16 * rt::kBM;     // weights of kDecode
 constexpr int64_t kDecodeOnceLarge = int64_t(1) << 23;
 std::atomic<int> g_decode_once{R97Q_DECODE_AUTO};
 // Whether a call takes the few-token path (qlinear_sm.h) where the choice is automatic: every call of at
-// most 128 tokens, and up to 1024 tokens while the products hold at most kSmWork steps of a
-// 128-token tile (16 for each CU) and a direction's partials stay within kSmPartBytes. Measured,
-// forward + backward, against the path for more tokens: 1 x 4096 x 4096 (tokens, outputs, inputs) 32 us
-// against 90, 128 x 1024 x 1024 25 against 71, 128 x 17408 x 5120 159 against 248, 256 x 4096 x 4096 76
-// against 105, 777 x 1408 x 2560 at rank 32 102 against 125, 1024 x 1024 x 1024 70 against 77; past
-// the line 300 x 4096 x 4096 at rank 32 (24 steps a CU) 123 against 118, 512 x 4096 x 4096 (32) 113 against
-// 106, 200 x 17408 x 5120 (85) 268 against 239.
-constexpr int64_t kSmAlwaysT = 128, kSmMaxT = 1024, kSmWork = 16 * 256, kSmPartBytes = int64_t(40) << 20;
-bool few_tokens(int64_t T, int64_t N, int64_t K) {
+// most 128 tokens, and up to 1024 tokens while the products hold few steps of a 128-token tile for each CU
+// and a direction's partials stay within kSmPartBytes. With an adapter that is 32 steps (the path for more
+// tokens takes three launches more a step), 20 without one, and 20 past 512 tokens at ranks 32 and 64, whose
+// up-projection the finishing launch runs as f32 FMAs. Measured, forward + backward, against the path
+// for more tokens: 1 x 4096 x 4096 (tokens, outputs, inputs) 32 us against 90, 128 x 17408 x 5120 142
+// against 248; rank 8 or 16: 512 x 4096 x 4096 (32 steps) 101 against 106, 1024 x 2048 x 4096 (32) 112 against
+// 116, 256 x 8192 x 4096 (32) 97 against 124; rank 64: 512 x 2048 x 8192 (32) 158 against 190, past 512
+// tokens 640 x 2048 x 4096 (20) 130 against 168, 1024 x 3072 x 2048 (24) 147 against 144, 1024 x 4096 x
+// 2048 (32) 183 against 158; rank 0: 256 x 5120 x 4096 (20) 66 against 74, 300 x 4096 x 4096 (24) 86
+// against 74.
+constexpr int64_t kSmAlwaysT = 128, kSmMaxT = 1024, kSmCUs = 256, kSmPartBytes = int64_t(40) << 20;
+bool few_tokens(int64_t T, int64_t N, int64_t K, int r) {
     if (T <= 0 || T > kSmMaxT || T * (N > K ? N : K) * 4 > kSmPartBytes) return false;
-    return T <= kSmAlwaysT || (T + 127) / 128 * (N / kBN) * (K / rt::kStep) <= kSmWork;
+    const int64_t steps = r > 0 && (r <= 16 || T <= 512) ? 32 : 20;
+    return T <= kSmAlwaysT || (T + 127) / 128 * (N / kBN) * (K / rt::kStep) <= steps * kSmCUs;
 }
 Shape shape(int64_t T, int64_t N, int64_t K, int r) {
     const int m = g_decode_once.load(std::memory_order_relaxed);
     const bool once = m != R97Q_DECODE_AUTO ? m == R97Q_DECODE_ONCE
                                             : T >= kDecodeOnceMinT || (T >= kDecodeOnceMinTLarge && N * K >= kDecodeOnceLarge);
-    return Shape{T, N, K, r, once, m == R97Q_DECODE_AUTO && few_tokens(T, N, K)};
+    return Shape{T, N, K, r, once, m == R97Q_DECODE_AUTO && few_tokens(T, N, K, r)};
 }
 
 // Split-K of the fused kernel (rt::Params::ksplit, nfull). A launch holds tiles = ceil(T/512) x
@@ -281,11 +285,12 @@ int64_t bwd_total(const Shape& s) { return s.small ? sm_ws(s, false).total : bwd
 struct ShrinkWs {
     int64_t P, Pt, At, part, done, total;
 };
-// Whether the adapter's adjoints on their own run as the few-token path's launches (f32 FMAs, the
-// partial sums few): measured, expand + shrink, at 32 tokens x 2048 columns x rank 16 23 us against 32, 256 x
-// 12288 x 16 30 against 53, 512 x 12288 x 16 57 against 58, 256 x 12288 x 64 102 against 111; past the
-// line 1024 x 2048 x 16 45 against 42, 512 x 12288 x 64 176 against 136.
-bool few_adapter(int64_t T, int r) { return T <= (r <= 16 ? 512 : 256); }
+// Whether the adapter's adjoints on their own run as the few-token path's launches (f32, the partial sums
+// few): measured, expand + shrink (tokens x columns x rank): 32 x 2048 x 16 23 us against 32, 1024 x 12288 x 16
+// 55 against 62, 1024 x 17408 x 16 66 against 76, 768 x 12288 x 32 70 against 78, 512 x 17408 x 64 115 against
+// 125; past the line 2000 x 2048 x 16 72 against 60, 1024 x 4096 x 32 82 against 74, 768 x 17408 x 64 153
+// against 138.
+bool few_adapter(int64_t T, int r) { return T <= (r <= 16 ? 1024 : r <= 32 ? 768 : 512); }
 ShrinkWs shrink_ws(int64_t T, int64_t K, int r) {
     ShrinkWs w{};
     if (r == 0) return w;

@@ -57,6 +57,9 @@ CASES = [
     (128, 384, 384, 8, 4, 256, False, False),
     (129, 512, 768, 16, 5, 256, False, True),   # past the unconditional line, two token tiles
     (500, 640, 896, 64, 5, 128, True, False),
+    (512, 2048, 2048, 16, 5, 256, False, False),  # 8 steps a CU, and 32 for each below
+    (512, 4096, 4096, 32, 5, 256, False, False),
+    (1000, 2048, 4096, 8, 4, 256, True, True),
     (1024, 256, 512, 32, 3, 256, False, False),  # the most tokens
 ]
 
@@ -163,7 +166,8 @@ def test_stages_keep_their_operands(T, N, K, r):
 
 
 @pytest.mark.parametrize("T,C,r", [(1, 128, 8), (33, 640, 64), (256, 384, 64), (257, 384, 32), (512, 256, 16),
-                                   (513, 256, 16)])
+                                   (512, 128, 64), (513, 128, 64), (768, 256, 32), (769, 256, 32), (1024, 256, 16),
+                                   (1025, 256, 8)])
 @pytest.mark.parametrize("off", [False, True])
 def test_adapter_adjoints(T, C, r, off):
     """The adapter's adjoints on their own on both sides of the few-token line, the factors and dX in views
