@@ -1005,7 +1005,7 @@ int64_t grad_chunks(int64_t T, int64_t K, int64_t N, int r) {
     // measured slower at ranks 8 to 32, 27-40%: the chunks' partial sums), two at rank 64, whose tiles
     // are half as long (2048 + 8192 columns, 16384 tokens: 12 chunks 114 us, 6 chunks 130).
     const int64_t cols = grad_blocks(K) + grad_blocks(N);
-    int64_t chunks = (r == 64 ? 512 : 256) / cols;
+    int64_t chunks = cols > 0 ? (r == 64 ? 512 : 256) / cols : 1;  // no columns: a size query's
     const int64_t tiles = grad_ld(T) / 64;  // no chunk smaller than one 64-token tile
     if (chunks > tiles) chunks = tiles;
     return chunks < 1 ? 1 : chunks;

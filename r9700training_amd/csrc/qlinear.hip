@@ -78,7 +78,8 @@ std::atomic<int> g_decode_once{R97Q_DECODE_AUTO};
 // against 74.
 constexpr int64_t kSmAlwaysT = 128, kSmMaxT = 1024, kSmCUs = 256, kSmPartBytes = int64_t(40) << 20;
 bool few_tokens(int64_t T, int64_t N, int64_t K, int r) {
-    if (T <= 0 || T > kSmMaxT || T * (N > K ? N : K) * 4 > kSmPartBytes) return false;
+    // (a size query may ask about any shape: less than a tile is not this path's, and no product overflows)
+    if (T <= 0 || T > kSmMaxT || N < kBN || K < kBN || (N > K ? N : K) > kSmPartBytes / 4 / T) return false;
     const int64_t steps = r > 0 && (r <= 16 || T <= 512) ? 32 : 20;
     return T <= kSmAlwaysT || (T + 127) / 128 * (N / kBN) * (K / rt::kStep) <= steps * kSmCUs;
 }
