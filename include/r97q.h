@@ -252,7 +252,11 @@ int r97q_weight_from_decoded(const int8_t* codes, const uint16_t* scale, int64_t
 #define R97Q_DECODE_FUSED 2
 int32_t r97q_set_decode_once(int32_t mode);
 
-/* Workspace the forward / backward need at this shape (bytes, 256-aligned pieces inside). */
+/* Workspace the forward / backward need at this shape (bytes, 256-aligned pieces inside). The sizes do
+ * not grow steadily with T: a call of few tokens asks for the partial products of its path, up to
+ * 40 MiB and a little, which can be more than thousands of tokens need. A call handed less than that,
+ * but as much as the path for more tokens needs at its shape (one workspace for several batches, say),
+ * takes that path: the results then differ by the order of the f32 sums. */
 int64_t r97q_fwd_workspace_bytes(int64_t T, int64_t N, int64_t K, int32_t rank);
 int64_t r97q_bwd_workspace_bytes(int64_t T, int64_t N, int64_t K, int32_t rank);
 
@@ -299,8 +303,8 @@ int r97q_iqr_encode_trellis(const float* W, int64_t N, int64_t K, int32_t bits, 
  *
  * The two calls above are these stages in order on one stream; a caller may issue them itself
  * (to time, overlap or reorder them). The workspace carries the adapter's activations between the
- * stages of one direction, so every stage of a direction gets the same workspace. Each is the part
- * of the reference rows named beside it.
+ * stages of one direction, so every stage of a direction gets the same workspace, of the same stated
+ * size (it settles the path). Each is the part of the reference rows named beside it.
  *
  * Forward: t = X.A^T (f32 into t_out) and the adapter operand of the fused kernel
  *          (lora_shrink_twin, src/adjoint/host/lora.cpp:226-244), and X's tiled copy in the workspace

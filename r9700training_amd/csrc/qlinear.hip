@@ -104,7 +104,7 @@ Shape shape(int64_t T, int64_t N, int64_t K, int r) {
 // and epilogue ~3 us, and the partials cost their bytes written and read (S x split tiles x
 // 512 x 128 x 8; the writes overlap other workgroups' products) at ~10 TB/s plus ~4 us for the
 // added launch. A split needs at least 16 steps a range and must beat no split by 7%.
-// Deterministic in the shape, so a call's bits never depend on anything else.
+// Deterministic in the shape, so the bits of a call on this path never depend on anything else.
 constexpr int kSplitMax = 8;
 struct Split {
     int S;      // ranges a split tile's reduction is dealt over (1: no split)
@@ -244,17 +244,17 @@ int sm_ranges(int64_t T, int64_t outputs, int64_t red) {
     return (int)(S < 1 ? 1 : S > 64 ? 64 : S);
 }
 
-// Forward: part [S, T, N] | tpart [SD, T, r] f32, and between the stage entries u [T, r] f32 (s.t) | act
-// [T, K] bf16 (X, as the tiled copy of the path for more tokens holds it).
-// Backward: part [S, T, K] | tpart [SD, T, r] f32, and between the stage entries u [T, r] (dt) | ts [T, r]
-// (s.t) f32 | Ac [r, K] bf16 | act [T, N] bf16 (dY). `fused`: the bytes without the stages' part.
-// the down product's ranges: one for few steps or many token blocks, up to a step a wave of its
+// The down product's ranges: one for few steps or many token blocks, up to a step a wave of its
 // workgroups (the finishing launch's workgroups each add the ranges, over every token)
 int sm_down_ranges(int64_t T, int64_t red) {
     const int64_t waves = 8 * (T <= 128 ? 1 : (T + 127) / 128);
     const int64_t n = (red / rt::kStep + waves - 1) / waves;
     return (int)(n < 16 ? n : 16);
 }
+// Forward: part [S, T, N] | tpart [SD, T, r] f32, and between the stage entries u [T, r] f32 (s.t) | act
+// [T, K] bf16 (X, as the tiled copy of the path for more tokens holds it).
+// Backward: part [S, T, K] | tpart [SD, T, r] f32, and between the stage entries u [T, r] (dt) | ts [T, r]
+// (s.t) f32 | Ac [r, K] bf16 | act [T, N] bf16 (dY). `fused`: the bytes without the stages' part.
 struct SmWs {
     int S, SD;
     int64_t part, tpart, u, ts, Ac, act, fused, total;
@@ -400,6 +400,23 @@ int check_ws(int64_t have, int64_t need, const void* ws, const char* who) {
         return R97Q_EWORKSPACE;
     }
     return R97Q_OK;
+}
+
+// Checks a call's workspace and settles its path. The few-token path's partials can be larger than the
+// other path's buffers for many more tokens (1024 x 1024 at rank 8, forward: 17.0 MiB at 512 tokens,
+// 4.1 MiB at 2048), so a caller's one workspace for its largest batch may hold only the other path's
+// layout of a smaller one; that path then serves it. `staged`: the stage entries' layout -- every
+// stage of a direction is handed the same size, so all settle alike.
+int settle(Shape& s, bool fwd, bool staged, int64_t have, const void* ws, const char* who) {
+    int64_t few = INT64_MAX;
+    if (s.small) {
+        const SmWs w = sm_ws(s, fwd);
+        few = staged ? w.total : w.fused;
+        if (have >= few) return check_ws(have, few, ws, who);
+        s.small = false;
+    }
+    const int64_t need = fwd ? fwd_ws(s).total : bwd_ws(s).total;
+    return check_ws(have, need < few ? need : few, ws, who);
 }
 
 // ---------------------------------------------------------------- the few-token path
@@ -872,8 +889,8 @@ int r97q_lora_fwd_prep(int64_t T, int64_t N, int64_t K, const uint16_t* X, const
         set_error("%s: null X, or A or t_out with rank > 0", who);
         return R97Q_EINVAL;
     }
-    const Shape sh = shape(T, N, K, rank);
-    if (int e = check_ws(workspace_bytes, fwd_total(sh), workspace, who)) return e;
+    Shape sh = shape(T, N, K, rank);
+    if (int e = settle(sh, true, true, workspace_bytes, workspace, who)) return e;
     uint8_t* wsb = static_cast<uint8_t*>(workspace);
     if (sh.small) return sm_fwd_prep(sh, X, A, scale, t_out, wsb, (hipStream_t)stream);
     return fwd_prep(sh, X, A, scale, t_out, wsb, (hipStream_t)stream);
@@ -890,8 +907,8 @@ int r97q_qlinear_fwd_base(const R97qWeight* w, const uint16_t* X, int64_t T, con
         set_error("%s: null X / Y (or B with rank > 0), or T <= 0", who);
         return R97Q_EINVAL;
     }
-    const Shape sh = shape(T, w->rows, w->cols, rank);
-    if (int e = check_ws(workspace_bytes, fwd_total(sh), workspace, who)) return e;
+    Shape sh = shape(T, w->rows, w->cols, rank);
+    if (int e = settle(sh, true, true, workspace_bytes, workspace, who)) return e;
     uint8_t* wsb = static_cast<uint8_t*>(workspace);
     if (sh.small) return sm_fwd_base(w, sh, B, Y, y_dtype, wsb, (hipStream_t)stream);
     return fwd_base(w, sh, B, Y, y_dtype, wsb, (hipStream_t)stream);
@@ -913,8 +930,8 @@ int r97q_qlinear_lora_fwd(const R97qWeight* w, const uint16_t* X, int64_t T, con
         set_error("%s: rank %d needs A, B and t_out", who, (int)rank);
         return R97Q_EINVAL;
     }
-    const Shape sh = shape(T, w->rows, w->cols, rank);
-    if (int e = check_ws(workspace_bytes, fwd_total(sh), workspace, who)) return e;
+    Shape sh = shape(T, w->rows, w->cols, rank);
+    if (int e = settle(sh, true, false, workspace_bytes, workspace, who)) return e;
     uint8_t* wsb = static_cast<uint8_t*>(workspace);
     const hipStream_t s = (hipStream_t)stream;
     if (sh.small) return sm_fwd(w, sh, X, A, B, scale, Y, y_dtype, t_out, wsb, s);
@@ -935,8 +952,8 @@ int r97q_lora_bwd_prep(int64_t T, int64_t N, int64_t K, const uint16_t* dY, cons
         set_error("%s: null dY, or A, B or t with rank > 0", who);
         return R97Q_EINVAL;
     }
-    const Shape sh = shape(T, N, K, rank);
-    if (int e = check_ws(workspace_bytes, bwd_total(sh), workspace, who)) return e;
+    Shape sh = shape(T, N, K, rank);
+    if (int e = settle(sh, false, true, workspace_bytes, workspace, who)) return e;
     uint8_t* wsb = static_cast<uint8_t*>(workspace);
     if (sh.small) return sm_bwd_prep(sh, dY, A, B, t, scale, wsb, (hipStream_t)stream);
     return bwd_prep(sh, dY, A, B, t, scale, wsb, (hipStream_t)stream);
@@ -954,8 +971,8 @@ int r97q_lora_bwd_grads(int64_t T, int64_t N, int64_t K, const uint16_t* X, cons
         set_error("%s: dA needs X, dB needs dY", who);
         return R97Q_EINVAL;
     }
-    const Shape sh = shape(T, N, K, rank);
-    if (int e = check_ws(workspace_bytes, bwd_total(sh), workspace, who)) return e;
+    Shape sh = shape(T, N, K, rank);
+    if (int e = settle(sh, false, true, workspace_bytes, workspace, who)) return e;
     uint8_t* wsb = static_cast<uint8_t*>(workspace);
     if (sh.small) return sm_bwd_grads(sh, X, dY, dA, dB, wsb, (hipStream_t)stream);
     return bwd_grads(sh, X, dY, dA, dB, wsb, (hipStream_t)stream);
@@ -972,8 +989,8 @@ int r97q_qlinear_dx_base(const R97qWeight* w, const uint16_t* dY, int64_t T, int
         set_error("%s: null dY / dX or T <= 0", who);
         return R97Q_EINVAL;
     }
-    const Shape sh = shape(T, w->rows, w->cols, rank);
-    if (int e = check_ws(workspace_bytes, bwd_total(sh), workspace, who)) return e;
+    Shape sh = shape(T, w->rows, w->cols, rank);
+    if (int e = settle(sh, false, true, workspace_bytes, workspace, who)) return e;
     uint8_t* wsb = static_cast<uint8_t*>(workspace);
     if (sh.small) return sm_dx_base(w, sh, dX, dx_dtype, dx_accumulate, wsb, (hipStream_t)stream);
     return dx_base(w, sh, dX, dx_dtype, dx_accumulate, wsb, (hipStream_t)stream);
@@ -996,8 +1013,8 @@ int r97q_qlinear_lora_bwd(const R97qWeight* w, const uint16_t* X, const uint16_t
         set_error("%s: rank %d needs X, A, B and t", who, (int)rank);
         return R97Q_EINVAL;
     }
-    const Shape sh = shape(T, w->rows, w->cols, rank);
-    if (int e = check_ws(workspace_bytes, bwd_total(sh), workspace, who)) return e;
+    Shape sh = shape(T, w->rows, w->cols, rank);
+    if (int e = settle(sh, false, false, workspace_bytes, workspace, who)) return e;
     uint8_t* wsb = static_cast<uint8_t*>(workspace);
     const hipStream_t s = (hipStream_t)stream;
     if (sh.small)

@@ -100,6 +100,68 @@ def test_few_tokens_match_the_other_path(modes, T, N, K, r, bits, run, codes8, b
         assert torch.isfinite(a).all() and e <= (2 ** -8 if bf16 and i < 2 else 2e-5), (i, e)
 
 
+@pytest.mark.parametrize("N,K,r,most", [(1024, 1024, 8, 2048), (2048, 512, 64, 2048), (640, 896, 32, 4096),
+                                        (256, 256, 0, 1536)])
+@pytest.mark.parametrize("T", [1, 128, 777, 1024])
+def test_workspace_of_a_larger_batch(modes, N, K, r, most, T):
+    """One workspace sized for `most` tokens serves the smaller batches, which may ask for more than it:
+    the bits are the few-token path's where its layout fits and the other path's where not, for the
+    fused and the stage entries alike, and nothing past the stated bytes is written. Less than either
+    path needs is still refused."""
+    from r9700training_amd import R97Q_F32, R97qError, _ptr, _stream, check, lib
+    from r9700training_amd.qlinear import qlinear_lora_bwd, qlinear_lora_fwd
+
+    print(f"case workspace of {most} tokens, T={T} N={N} K={K} r={r}", flush=True)
+    rng = np.random.default_rng(T + N)
+    keep = []
+    w = _weight(N, K, 5, 128, False, T + N, keep)
+    X, dY = bf16_tensor(rng.standard_normal((T, K))), bf16_tensor(rng.standard_normal((T, N)))
+    A = bf16_tensor(0.01 * rng.standard_normal((r, K))) if r else None
+    B = bf16_tensor(0.01 * rng.standard_normal((N, r))) if r else None
+    L, P, st = lib(), _ptr, _stream()
+    kw = dict(dx_dtype=torch.float32)
+    modes(False)
+    need = [f(T, N, K, r) for f in (L.r97q_fwd_workspace_bytes, L.r97q_bwd_workspace_bytes)]
+    Yo, to = qlinear_lora_fwd(w, X, A, B, 2.0, y_dtype=torch.float32)
+    other = (Yo, *qlinear_lora_bwd(w, X, dY, A, B, to, 2.0, **kw))
+    modes(True)
+    Yf, tf = qlinear_lora_fwd(w, X, A, B, 2.0, y_dtype=torch.float32)
+    own = (Yf, *qlinear_lora_bwd(w, X, dY, A, B, to, 2.0, **kw))
+    asked = [f(T, N, K, r) for f in (L.r97q_fwd_workspace_bytes, L.r97q_bwd_workspace_bytes)]
+    held = [f(most, N, K, r) for f in (L.r97q_fwd_workspace_bytes, L.r97q_bwd_workspace_bytes)]
+    buf = [torch.full((max(h, n) + 4096,), 0xA5, dtype=torch.uint8, device="cuda") for h, n in zip(held, need)]
+    ws = [b[:h] for b, h in zip(buf, held)]
+    Y, t = qlinear_lora_fwd(w, X, A, B, 2.0, y_dtype=torch.float32, workspace=ws[0])
+    got = (Y, *qlinear_lora_bwd(w, X, dY, A, B, to, 2.0, workspace=ws[1], **kw))
+    Ys, dXs = torch.empty_like(Y), torch.empty_like(got[1])
+    ts = torch.empty_like(t) if r else None
+    dAs, dBs = (torch.zeros_like(got[2]), torch.zeros_like(got[3])) if r else (None, None)
+    f, b = (P(ws[0]), held[0], st), (P(ws[1]), held[1], st)
+    check(L.r97q_lora_fwd_prep(T, N, K, P(X), P(A), r, 2.0, P(ts), *f), "fwd_prep")
+    check(L.r97q_qlinear_fwd_base(C.byref(w.w), P(X), T, P(B), r, P(Ys), R97Q_F32, *f), "fwd_base")
+    check(L.r97q_lora_bwd_prep(T, N, K, P(dY), P(A), P(B), P(to), r, 2.0, *b), "bwd_prep")
+    check(L.r97q_lora_bwd_grads(T, N, K, P(X), P(dY), r, P(dAs), P(dBs), *b), "bwd_grads")
+    check(L.r97q_qlinear_dx_base(C.byref(w.w), P(dY), T, r, P(dXs), R97Q_F32, 0, *b), "dx_base")
+    torch.cuda.synchronize()
+    for bb, h in zip(buf, held):
+        assert (bb[h:] == 0xA5).all()
+    staged = (Ys, dXs, dAs, dBs)
+    for i in range(4 if r else 2):
+        one = 0 if i == 0 else 1
+        assert torch.equal(got[i], own[i]) or torch.equal(got[i], other[i]), i
+        assert torch.equal(staged[i], own[i]) or torch.equal(staged[i], other[i]), i
+        if held[one] >= asked[one]:
+            assert torch.equal(got[i], own[i]) and torch.equal(staged[i], own[i]), i
+    for one, short in enumerate(min(n, a) for n, a in zip(need, asked)):
+        with pytest.raises(R97qError):
+            # the fused entries need no more than the stages' part past the partials
+            small = buf[one][: short // 8]
+            if one == 0:
+                qlinear_lora_fwd(w, X, A, B, 2.0, workspace=small)
+            else:
+                qlinear_lora_bwd(w, X, dY, A, B, to, 2.0, workspace=small)
+
+
 @pytest.mark.parametrize("over", ["X", "dY"])
 @pytest.mark.parametrize("T,r", [(5, 8), (130, 16), (300, 64)])
 def test_outputs_over_their_inputs(T, r, over):
