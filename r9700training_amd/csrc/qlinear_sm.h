@@ -83,8 +83,8 @@ struct Finish {
     float tscale;
     int64_t N;
     float* dB;
-    // what a later stage reads: ts [T, r] = tscale * t, and copies of bf16 operands (n a multiple of 8;
-    // null `to`: none)
+    // what a later stage reads: ts [T, r] = tscale * t, and copies of bf16 operands (n a multiple of 8, `to`
+    // on 16 bytes, `from` anywhere; null `to`: none)
     float* ts;
     struct Copy {
         const uint16_t* from;

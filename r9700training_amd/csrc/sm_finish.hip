@@ -288,8 +288,19 @@ __global__ __launch_bounds__(kThreads, R <= 32 ? 4 : 2) void sm_finish_kernel(co
     }
     const Finish::Copy& c = f.copy[b < n.copies[0] ? 0 : 1];
     if (b >= n.copies[0]) b -= n.copies[0];
-    for (int64_t i = (int64_t)b * kCopy + 8 * threadIdx.x; i < c.n && i < (int64_t)(b + 1) * kCopy; i += 8 * kThreads)
-        *reinterpret_cast<uint4*>(c.to + i) = *reinterpret_cast<const uint4*>(c.from + i);
+    // (A as the caller holds it may lie off 16 bytes: a value at a time)
+    const bool vec = (reinterpret_cast<uintptr_t>(c.from) & 15) == 0;
+    for (int64_t i = (int64_t)b * kCopy + 8 * threadIdx.x; i < c.n && i < (int64_t)(b + 1) * kCopy; i += 8 * kThreads) {
+        uint4 v;
+        if (vec) {
+            v = *reinterpret_cast<const uint4*>(c.from + i);
+        } else {
+            const uint16_t* p = c.from + i;
+            v = uint4{(uint32_t)p[0] | (uint32_t)p[1] << 16, (uint32_t)p[2] | (uint32_t)p[3] << 16,
+                      (uint32_t)p[4] | (uint32_t)p[5] << 16, (uint32_t)p[6] | (uint32_t)p[7] << 16};
+        }
+        *reinterpret_cast<uint4*>(c.to + i) = v;
+    }
 }
 
 }  // namespace

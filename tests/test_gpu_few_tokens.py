@@ -227,6 +227,41 @@ def test_stages_keep_their_operands(T, N, K, r):
         assert torch.equal(t, ts) and torch.equal(dA, dAs) and torch.equal(dB, dBs) and torch.equal(t, tn)
 
 
+@pytest.mark.parametrize("T,N,K,r", [(1, 384, 512, 8), (33, 256, 640, 32), (130, 256, 384, 16), (300, 512, 256, 64)])
+def test_factor_off_its_alignment(T, N, K, r):
+    """A in a view one, two or four elements past an aligned start (off 16 bytes, the last on 8): the fused
+    entries, the stages and the forward that allocates nothing read it a value or half a piece at a
+    time, the aligned A's bits."""
+    from r9700training_amd import R97Q_F32, _ptr, _stream, check, lib
+    from r9700training_amd.qlinear import bwd_workspace, qlinear_lora_bwd, qlinear_lora_fwd
+
+    print(f"case few tokens unaligned A T={T} N={N} K={K} r={r}", flush=True)
+    rng = np.random.default_rng(T)
+    keep = []
+    w = _weight(N, K, 5, 128, False, T, keep)
+    X, dY = bf16_tensor(rng.standard_normal((T, K))), bf16_tensor(rng.standard_normal((T, N)))
+    A, B = bf16_tensor(0.01 * rng.standard_normal((r, K))), bf16_tensor(0.01 * rng.standard_normal((N, r)))
+    L, P, st = lib(), _ptr, _stream()
+    Y, t = qlinear_lora_fwd(w, X, A, B, 2.0, y_dtype=torch.float32)
+    want = (Y, t, *qlinear_lora_bwd(w, X, dY, A, B, t, 2.0, dx_dtype=torch.float32))
+    for at in (1, 2, 4):
+        Au = torch.empty(r * K + 8, dtype=torch.bfloat16, device="cuda")[at:][: r * K].view(r, K).copy_(A)
+        Y2, t2 = qlinear_lora_fwd(w, X, Au, B, 2.0, y_dtype=torch.float32)
+        got = (Y2, t2, *qlinear_lora_bwd(w, X, dY, Au, B, t, 2.0, dx_dtype=torch.float32))
+        Yn, tn = torch.empty_like(Y), torch.empty_like(t)
+        check(L.r97q_qlinear_lora_fwd_noalloc(C.byref(w.w), P(X), T, P(Au), P(B), r, 2.0, P(Yn), R97Q_F32, P(tn), st),
+              "noalloc")
+        ws = bwd_workspace(T, N, K, r)
+        b = (P(ws), ws.numel(), st)
+        dX, dA, dB = torch.empty_like(want[2]), torch.zeros_like(want[3]), torch.zeros_like(want[4])
+        check(L.r97q_lora_bwd_prep(T, N, K, P(dY), P(Au), P(B), P(t), r, 2.0, *b), "bwd_prep")
+        check(L.r97q_lora_bwd_grads(T, N, K, P(X), P(dY), r, P(dA), P(dB), *b), "bwd_grads")
+        check(L.r97q_qlinear_dx_base(C.byref(w.w), P(dY), T, r, P(dX), R97Q_F32, 0, *b), "dx_base")
+        torch.cuda.synchronize()
+        for i, (g, x) in enumerate(zip((*got, Yn, tn, dX, dA, dB), (*want, *want))):
+            assert torch.equal(g, x), (at, i)
+
+
 @pytest.mark.parametrize("T,C,r", [(1, 128, 8), (33, 640, 64), (256, 384, 64), (257, 384, 32), (512, 256, 16),
                                    (512, 128, 64), (513, 128, 64), (768, 256, 32), (769, 256, 32), (1024, 256, 16),
                                    (1025, 256, 8)])
