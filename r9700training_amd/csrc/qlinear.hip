@@ -514,6 +514,11 @@ int sm_fwd_base(const R97qWeight* w, const Shape& sh, const uint16_t* B, void* Y
     return sm::launch_finish(f, s);
 }
 
+bool overlap(const void* p, int64_t p_bytes, const void* q, int64_t q_bytes) {
+    const uintptr_t a = reinterpret_cast<uintptr_t>(p), b = reinterpret_cast<uintptr_t>(q);
+    return p && q && a < b + q_bytes && b < a + p_bytes;
+}
+
 int sm_bwd(const R97qWeight* w, const Shape& sh, const uint16_t* X, const uint16_t* dY, const uint16_t* A,
            const uint16_t* B, float scale, const float* t, void* dX, int32_t dx_dtype, int32_t accumulate, float* dA,
            float* dB, uint8_t* wsb, hipStream_t s) {
@@ -528,12 +533,10 @@ int sm_bwd(const R97qWeight* w, const Shape& sh, const uint16_t* X, const uint16
     f.tscale = scale;
     f.N = sh.N;
     f.dB = dB;
-    // dX written over dY or X (as the path for more tokens allows): the gradients read them first
-    const auto over = [&](const void* in, int64_t bytes) {
-        const uintptr_t a = reinterpret_cast<uintptr_t>(dX), b = reinterpret_cast<uintptr_t>(in);
-        return in && a < b + bytes && b < a + sh.T * sh.K * (f.out_f32 ? 4 : 2);
-    };
-    if ((dA && over(X, sh.T * sh.K * 2)) || (dB && over(dY, sh.T * sh.N * 2))) {
+    // dX written over dY, X or t (as the path for more tokens allows): the gradients read them first
+    const int64_t dx_bytes = sh.T * sh.K * (f.out_f32 ? 4 : 2);
+    if ((dA && overlap(dX, dx_bytes, X, sh.T * sh.K * 2)) ||
+        (dB && (overlap(dX, dx_bytes, dY, sh.T * sh.N * 2) || overlap(dX, dx_bytes, t, sh.T * sh.r * 4)))) {
         f.out = nullptr;
         if (int e = sm::launch_finish(f, s)) return e;
         f.out = dX;

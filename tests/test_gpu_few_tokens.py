@@ -187,6 +187,28 @@ def test_outputs_over_their_inputs(T, r, over):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("T,r", [(5, 8), (130, 16), (300, 64)])
+def test_dx_over_t(T, r):
+    """An f32 dX whose buffer holds t: the separate buffers' bits, as on the path for more tokens."""
+    from r9700training_amd.qlinear import qlinear_lora_bwd, qlinear_lora_fwd
+
+    print(f"case few tokens dX over t T={T} r={r}", flush=True)
+    rng = np.random.default_rng(T)
+    keep = []
+    N, K = 512, 384
+    w = _weight(N, K, 5, 128, False, T, keep)
+    X, dY = bf16_tensor(rng.standard_normal((T, K))), bf16_tensor(rng.standard_normal((T, N)))
+    A, B = bf16_tensor(0.01 * rng.standard_normal((r, K))), bf16_tensor(0.01 * rng.standard_normal((N, r)))
+    _, t = qlinear_lora_fwd(w, X, A, B, 2.0)
+    want = qlinear_lora_bwd(w, X, dY, A, B, t, 2.0, dx_dtype=torch.float32)
+    dX = torch.empty_like(want[0])
+    t2 = dX.view(-1)[: T * r].view(T, r).copy_(t)
+    got = qlinear_lora_bwd(w, X, dY, A, B, t2, 2.0, dX=dX)
+    torch.cuda.synchronize()
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("T,N,K,r", [(7, 384, 512, 16), (130, 256, 384, 0), (300, 512, 256, 64)])
 def test_stages_keep_their_operands(T, N, K, r):
     """The stage entries on this path: the fused entries' bits, with X and dY overwritten between the
