@@ -1174,7 +1174,9 @@ int r97q_lora_shrink_bwd(int64_t T, int64_t K, const uint16_t* X, const uint16_t
     if (int e = check_ws(workspace_bytes, ws.total, workspace, who)) return e;
     uint8_t* wsb = static_cast<uint8_t*>(workspace);
     const hipStream_t s = (hipStream_t)stream;
-    if (few_adapter(T, rank)) {  // one launch: dX and dA from the f32 t_cot
+    // one launch: dX and dA from the f32 t_cot (a dX written over t_cot or A takes the launches below, which
+    // read both before they write it)
+    if (few_adapter(T, rank) && !overlap(dX, T * K * 4, t_cot, T * rank * 4) && !overlap(dX, T * K * 4, A, rank * K * 2)) {
         sm::Finish f{};
         f.T = T;
         f.rank = rank;

@@ -315,3 +315,28 @@ def test_adapter_adjoints(T, C, r, off):
     for got, ref in ((t_cot, want), (dB, 2.0 * (x.T @ t.double())), (dX, dX0.double() + tc @ a), (dX2, tc @ a),
                      (dA, tc.T @ x)):
         assert _rel(got, ref) <= 2e-5, _rel(got, ref)
+
+
+@pytest.mark.parametrize("T,K,r", [(5, 128, 64), (300, 384, 16), (1025, 256, 8)])
+def test_shrink_dx_over_its_inputs(T, K, r):
+    """The shrink's f32 dX in a buffer that holds t_cot, or A: written after both are read, on either side
+    of the few-token line. Against float64 products, with the bound above."""
+    from r9700training_amd.qlinear import lora_shrink_bwd
+
+    print(f"case shrink dX over its inputs T={T} K={K} r={r}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(T)
+    u = torch.randn((T, r), generator=g, device="cuda")
+    A = torch.randn((r, K), generator=g, device="cuda").to(torch.bfloat16)
+    X = torch.randn((T, K), generator=g, device="cuda").to(torch.bfloat16)
+    want = (u.double() @ A.double(), u.double().T @ X.double())
+    for over in ("t_cot", "A"):
+        dX = torch.empty((max(T, r), K), device="cuda")  # room for A at its start
+        at, cot = A, u
+        if over == "t_cot":
+            cot = dX.view(-1)[: T * r].view(T, r).copy_(u)
+        else:
+            at = dX.view(torch.bfloat16).view(-1)[: r * K].view(r, K).copy_(A)
+        got = lora_shrink_bwd(X, at, cot, dX=dX[:T])
+        torch.cuda.synchronize()
+        for a, b in zip(got, want):
+            assert _rel(a, b) <= 2e-5, (over, _rel(a, b))
