@@ -1123,6 +1123,12 @@ int r97q_lora_shrink_q_bwd(int64_t T, int64_t K, const void* a, int32_t a_dtype,
     // the two cotangents, one for dA; the others through the values g and x
     const int8_t* codes = code_f32 || reinterpret_cast<uintptr_t>(a) % 16 != 0 ? nullptr : static_cast<const int8_t*>(a);
     const bool up = codes && coded_up_takes(gw, K, groups), grads = codes && grads_coded_takes(gw, K, groups);
+    // (dA first: it reads t_cot itself, which da or ds may be written over)
+    if (dA && grads) {
+        if (int e = launch_grads_coded(rank, t_cot, codes, a_scale, T, K, groups, gw, dA,
+                                       reinterpret_cast<float*>(wsb + ws.part), done, s))
+            return e;
+    }
     if ((da || ds) && up) {
         if (int e = launch_coded_up(P, At, codes, a_scale, T, K, groups, gw, rank, da, ds, s)) return e;
     } else if (da || ds) {
@@ -1131,10 +1137,7 @@ int r97q_lora_shrink_q_bwd(int64_t T, int64_t K, const void* a, int32_t a_dtype,
         if (int e = launch_lora_up(P, At, T, K, rank, g, 0, s)) return e;
         if (int e = launch_coded_cot(g, a, code_f32, a_scale, T, K, groups, gw, da, ds, s)) return e;
     }
-    if (dA && grads)
-        return launch_grads_coded(rank, t_cot, codes, a_scale, T, K, groups, gw, dA, reinterpret_cast<float*>(wsb + ws.part),
-                                  done, s);
-    if (dA) {
+    if (dA && !grads) {
         // dA += t_cot^T . x with x = [hi | lo](a * a_scale): two gradient passes, one a half
         uint16_t* xhi = reinterpret_cast<uint16_t*>(wsb + ws.xhi);
         uint16_t* xlo = reinterpret_cast<uint16_t*>(wsb + ws.xlo);

@@ -258,6 +258,29 @@ def test_int8_codes_match_the_general_path(T, K, gw, r):
     assert torch.equal(only[1], out[0][1])
 
 
+@pytest.mark.parametrize("T,K,gw,r", [(5, 128, 64, 8), (200, 768, 256, 64), (129, 1024, 512, 16), (64, 896, 96, 16)])
+def test_coded_shrink_da_over_t_cot(T, K, gw, r):
+    """da added into the buffer that holds t_cot: t_cot is read first, whichever kernels the group width
+    takes -- the separate buffers' bits, plus t_cot."""
+    from r9700training_amd.qlinear import lora_shrink_q_bwd
+
+    print(f"case coded shrink da over t_cot T={T} K={K} gw={gw} r={r}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(T + K)
+    groups = (K + gw - 1) // gw
+    code = torch.randint(-128, 128, (T, K), generator=g, device="cuda", dtype=torch.int8)
+    s = 0.01 + torch.rand((T, groups), generator=g, device="cuda")
+    A = (0.1 * torch.randn((r, K), generator=g, device="cuda")).to(torch.bfloat16)
+    t = torch.randn((T, r), generator=g, device="cuda")
+    base = torch.zeros(T * K, device="cuda")
+    base[: T * r] = t.view(-1)
+    want = lora_shrink_q_bwd(code, s, A, t, da=base.clone().view(T, K), group_width=gw)
+    da = base.clone()
+    got = lora_shrink_q_bwd(code, s, A, da[: T * r].view(T, r), da=da.view(T, K), group_width=gw)
+    torch.cuda.synchronize()
+    for i, (a, b) in enumerate(zip(got, want)):
+        assert torch.equal(a, b), i
+
+
 @pytest.mark.parametrize("T,N,K,bf16", [(1, 128, 128, False), (31, 256, 640, True), (33, 384, 1152, False),
                                         (100, 8192, 128, False), (130, 6528, 256, False), (129, 128, 4224, False)])
 def test_coded_forward_few_tokens(T, N, K, bf16):
