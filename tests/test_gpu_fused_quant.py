@@ -114,6 +114,48 @@ def test_lane_kernels_equal_the_general_ones(part, dtype, rows, n, group):
     assert np.array_equal(y.view(torch.int16).cpu().numpy().view(np.uint16), _bf16_of(wy))
 
 
+@pytest.mark.parametrize("part", ["silu_mul", "sigmoid_mul"])
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+def test_lane_sigmoid_at_its_extremes(part, dtype):
+    """Gate values where 1 + exp(-x) is infinite, its reciprocal subnormal, 1 or as good as 1, and infinities
+    and NaN, each in a group of its own beside ordinary ones: the general kernels' codes, scales, outputs
+    and gradients, NaN where they have NaN."""
+    from r9700training_amd.quant import fused_had_quant_i8g, fused_had_quant_i8g_bwd
+
+    print(f"case fused lanes extremes {part} {dtype}", flush=True)
+    group = 32
+    gates = [-708.0, -708.5, -709.0, -709.5, -709.78, -710.0, -744.0, -746.0, -1e4, -1e38, 1e4, 1e38, 37.0, 709.0,
+             float("inf"), float("-inf"), float("nan"), 1e-39, -0.0]
+    n, rows = group * len(gates), 3
+    rng, x0, x1, d0, d1 = _inputs(part, rows, n, dtype, 11)
+    for i, v in enumerate(gates):
+        d0[0, i * group] = v                          # one among ordinary values
+        d0[1, i * group:(i + 1) * group] = v          # the whole group
+        d0[2, i * group:(i + 1) * group:3] = v
+
+    def off(t):
+        return None if t is None else torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda")[1:].view(t.shape).copy_(t)
+
+    codes, scale, y = fused_had_quant_i8g(part, d0, d1, group, want_y=True)
+    codes_g, scale_g, y_g = fused_had_quant_i8g(part, off(d0), off(d1), group, want_y=True)
+    rnd = lambda shape: torch.tensor(rng.standard_normal(shape), dtype=torch.float32, device="cuda")  # noqa: E731
+    g, go, b0, b1 = rnd((rows, n)), rnd((rows, n)), rnd(tuple(d0.shape)), rnd((rows, n))
+    got = fused_had_quant_i8g_bwd(part, d0, d1, group, scale, g, go, dx0=b0.clone(), dx1=b1.clone())
+    gen = fused_had_quant_i8g_bwd(part, off(d0), off(d1), group, scale, off(g), off(go), dx0=off(b0), dx1=off(b1))
+    torch.cuda.synchronize()
+    pairs = [("codes", codes, codes_g), ("scale", scale, scale_g), ("y", y, y_g), ("dx0", got[0], gen[0])]
+    if part == "sigmoid_mul":
+        pairs.append(("dx1", got[1], gen[1]))
+    bad = []
+    for name, a, b in pairs:
+        a, b = a.double(), b.double()
+        same = (a == b) | (a.isnan() & b.isnan())
+        if not same.all():
+            where = (~same).nonzero()[:6].tolist()
+            bad.append((name, int((~same).sum()), [(w, a[tuple(w)].item(), b[tuple(w)].item()) for w in where]))
+    assert not bad, bad
+
+
 @pytest.mark.parametrize("part", ["rmsnorm", "silu_mul", "sigmoid_mul"])
 def test_fused_mask_engaged(part):
     """A scale below the forward's (as a tape's cotangent may arrive against) clamps part of every
