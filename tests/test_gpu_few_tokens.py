@@ -249,6 +249,35 @@ def test_stages_keep_their_operands(T, N, K, r):
         assert torch.equal(t, ts) and torch.equal(dA, dAs) and torch.equal(dB, dBs) and torch.equal(t, tn)
 
 
+@pytest.mark.parametrize("T", [40, 1100])
+def test_backward_without_gradients(T):
+    """Both factor gradients skipped (NULL) with an adapter: dX is the bits it is with them, on either path,
+    from the fused and the stage entries."""
+    from r9700training_amd import R97Q_F32, _ptr, _stream, check, lib
+    from r9700training_amd.qlinear import bwd_workspace, qlinear_lora_bwd, qlinear_lora_fwd
+
+    print(f"case backward without gradients T={T}", flush=True)
+    rng = np.random.default_rng(T)
+    keep = []
+    N, K, r = 256, 384, 16
+    w = _weight(N, K, 5, 128, False, T, keep)
+    X, dY = bf16_tensor(rng.standard_normal((T, K))), bf16_tensor(rng.standard_normal((T, N)))
+    A, B = bf16_tensor(0.01 * rng.standard_normal((r, K))), bf16_tensor(0.01 * rng.standard_normal((N, r)))
+    L, P, st = lib(), _ptr, _stream()
+    _, t = qlinear_lora_fwd(w, X, A, B, 2.0)
+    want = qlinear_lora_bwd(w, X, dY, A, B, t, 2.0, dx_dtype=torch.float32)[0]
+    ws = bwd_workspace(T, N, K, r)
+    b = (P(ws), ws.numel(), st)
+    dX, dXs = torch.empty_like(want), torch.empty_like(want)
+    check(L.r97q_qlinear_lora_bwd(C.byref(w.w), P(X), P(dY), T, P(A), P(B), r, 2.0, P(t), P(dX), R97Q_F32, 0, None, None, *b),
+          "bwd")
+    check(L.r97q_lora_bwd_prep(T, N, K, P(dY), P(A), P(B), P(t), r, 2.0, *b), "bwd_prep")
+    check(L.r97q_lora_bwd_grads(T, N, K, P(X), P(dY), r, None, None, *b), "bwd_grads")
+    check(L.r97q_qlinear_dx_base(C.byref(w.w), P(dY), T, r, P(dXs), R97Q_F32, 0, *b), "dx_base")
+    torch.cuda.synchronize()
+    assert torch.equal(dX, want) and torch.equal(dXs, want)
+
+
 @pytest.mark.parametrize("T,N,K,r", [(1, 384, 512, 8), (33, 256, 640, 32), (130, 256, 384, 16), (300, 512, 256, 64)])
 def test_factor_off_its_alignment(T, N, K, r):
     """A in a view one, two or four elements past an aligned start (off 16 bytes, the last on 8): the fused
