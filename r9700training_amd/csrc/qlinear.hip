@@ -45,7 +45,8 @@ struct Shape {
     int64_t T, N, K;
     int r;
     bool once;
-    bool small;  // the few-token path (qlinear_sm.h)
+    bool small_fwd, small_bwd;  // the direction takes the few-token path (qlinear_sm.h)
+    bool& small(bool fwd) { return fwd ? small_fwd : small_bwd; }
 };
 
 // The base products either decode each weight tile in the main loop, once for every 512-token
@@ -65,29 +66,40 @@ constexpr int64_t kDecodeOnceMinT = 32 * rt::kBM;          // any weight from 16
 constexpr int64_t kDecodeOnceMinTLarge = 16 * rt::kBM;     // weights of kDecodeOnceLarge values from 8192
 constexpr int64_t kDecodeOnceLarge = int64_t(1) << 23;
 std::atomic<int> g_decode_once{R97Q_DECODE_AUTO};
-// Whether a call takes the few-token path (qlinear_sm.h) where the choice is automatic: every call of at
-// most 128 tokens, and up to 1024 tokens while the products hold few steps of a 128-token tile for each CU
-// and a direction's partials stay within kSmPartBytes. With an adapter that is 32 steps (the path for more
-// tokens takes three launches more a step), 20 without one, and 20 past 512 tokens at ranks 32 and 64, whose
-// up-projection the finishing launch runs as f32 FMAs. Measured, forward + backward, against the path
-// for more tokens: 1 x 4096 x 4096 (tokens, outputs, inputs) 32 us against 90, 128 x 17408 x 5120 142
-// against 248; rank 8 or 16: 512 x 4096 x 4096 (32 steps) 101 against 106, 1024 x 2048 x 4096 (32) 112 against
-// 116, 256 x 8192 x 4096 (32) 97 against 124; rank 64: 512 x 2048 x 8192 (32) 158 against 190, past 512
-// tokens 640 x 2048 x 4096 (20) 130 against 168, 1024 x 3072 x 2048 (24) 147 against 144, 1024 x 4096 x
-// 2048 (32) 183 against 158; rank 0: 256 x 5120 x 4096 (20) 66 against 74, 300 x 4096 x 4096 (24) 86
-// against 74.
+// Whether a direction of a call (a product of `outs` outputs over a reduction of `red`) takes the
+// few-token path (qlinear_sm.h) where the choice is automatic: up to 128 tokens, and up to 1024 while
+// the products hold few steps of a 128-token tile for each CU and a direction's partials stay within
+// kSmPartBytes. With an adapter that is 32 steps (the path for more tokens takes three launches more a
+// step), 20 without one, and 20 past 512 tokens at ranks 32 and 64, whose up-projection the finishing
+// launch runs as f32 FMAs. Measured, forward + backward, against the path for more tokens:
+// 1 x 4096 x 4096 (tokens, outputs, inputs) 32 us against 90, 128 x 17408 x 5120 142 against 248; rank 8
+// or 16: 512 x 4096 x 4096 (32 steps) 101 against 106, 1024 x 2048 x 4096 (32) 112 against 116, 256 x 8192 x
+// 4096 (32) 97 against 124; rank 64: 512 x 2048 x 8192 (32) 158 against 190, past 512 tokens 640 x 2048 x
+// 4096 (20) 130 against 168, 1024 x 3072 x 2048 (24) 147 against 144, 1024 x 4096 x 2048 (32) 183 against 158;
+// rank 0: 256 x 5120 x 4096 (20) 66 against 74, 300 x 4096 x 4096 (24) 86 against 74.
+// And while the finishing launch's work -- every output value, in the forward with its r FMAs -- is small
+// beside the reduction whose steps the split deals out: many outputs of a short reduction cost more to
+// finish than the whole product of the other path takes. (The other path's backward with an adapter has
+// the gradients' partial sums to add besides.) Over 1260 random shapes within the lines above the
+// forward is more than 3% slower than that path at 114 without this line (773 x 9984 x 128, rank 64: 98 us
+// against 30; 497 x 7808 x 512, rank 64: 62 against 35; 814 x 5504 x 896, rank 16: 45 against 36) and at 19
+// with it, the backward at 26 (846 x 256 x 9984, rank 8: 48 against 38) and at 4; 3 of these directions take
+// the other path and lose more than 3% by it.
 constexpr int64_t kSmAlwaysT = 128, kSmMaxT = 1024, kSmCUs = 256, kSmPartBytes = int64_t(40) << 20;
-bool few_tokens(int64_t T, int64_t N, int64_t K, int r) {
+bool few_tokens(int64_t T, int64_t N, int64_t K, int r, bool fwd) {
     // (a size query may ask about any shape: less than a tile is not this path's, and no product overflows)
     if (T <= 0 || T > kSmMaxT || N < kBN || K < kBN || (N > K ? N : K) > kSmPartBytes / 4 / T) return false;
     const int64_t steps = r > 0 && (r <= 16 || T <= 512) ? 32 : 20;
-    return T <= kSmAlwaysT || (T + 127) / 128 * (N / kBN) * (K / rt::kStep) <= steps * kSmCUs;
+    if (T > kSmAlwaysT && (T + 127) / 128 * (N / kBN) * (K / rt::kStep) > steps * kSmCUs) return false;
+    if (fwd) return T * N / 64 * (64 + r) <= 2000000 + 2000 * K;
+    return T * K <= (r > 0 ? 2 : 1) * (2000000 + 2000 * N);
 }
 Shape shape(int64_t T, int64_t N, int64_t K, int r) {
     const int m = g_decode_once.load(std::memory_order_relaxed);
     const bool once = m != R97Q_DECODE_AUTO ? m == R97Q_DECODE_ONCE
                                             : T >= kDecodeOnceMinT || (T >= kDecodeOnceMinTLarge && N * K >= kDecodeOnceLarge);
-    return Shape{T, N, K, r, once, m == R97Q_DECODE_AUTO && few_tokens(T, N, K, r)};
+    const bool small = m == R97Q_DECODE_AUTO;
+    return Shape{T, N, K, r, once, small && few_tokens(T, N, K, r, true), small && few_tokens(T, N, K, r, false)};
 }
 
 // Split-K of the fused kernel (rt::Params::ksplit, nfull). A launch holds tiles = ceil(T/512) x
@@ -274,8 +286,8 @@ SmWs sm_ws(const Shape& s, bool fwd) {
     return w;
 }
 
-int64_t fwd_total(const Shape& s) { return s.small ? sm_ws(s, true).total : fwd_ws(s).total; }
-int64_t bwd_total(const Shape& s) { return s.small ? sm_ws(s, false).total : bwd_ws(s).total; }
+int64_t fwd_total(const Shape& s) { return s.small_fwd ? sm_ws(s, true).total : fwd_ws(s).total; }
+int64_t bwd_total(const Shape& s) { return s.small_bwd ? sm_ws(s, false).total : bwd_ws(s).total; }
 
 // The adapter rows on their own (the shrink's and the expand's adjoints), workspace layouts:
 // shrink: P [T, 2r] | Pt [2r, ldt] | At [K, r] | part [chunks, r, K] | done
@@ -409,11 +421,11 @@ int check_ws(int64_t have, int64_t need, const void* ws, const char* who) {
 // stage of a direction is handed the same size, so all settle alike.
 int settle(Shape& s, bool fwd, bool staged, int64_t have, const void* ws, const char* who) {
     int64_t few = INT64_MAX;
-    if (s.small) {
+    if (s.small(fwd)) {
         const SmWs w = sm_ws(s, fwd);
         few = staged ? w.total : w.fused;
         if (have >= few) return check_ws(have, few, ws, who);
-        s.small = false;
+        s.small(fwd) = false;
     }
     const int64_t need = fwd ? fwd_ws(s).total : bwd_ws(s).total;
     return check_ws(have, need < few ? need : few, ws, who);
@@ -895,7 +907,7 @@ int r97q_lora_fwd_prep(int64_t T, int64_t N, int64_t K, const uint16_t* X, const
     Shape sh = shape(T, N, K, rank);
     if (int e = settle(sh, true, true, workspace_bytes, workspace, who)) return e;
     uint8_t* wsb = static_cast<uint8_t*>(workspace);
-    if (sh.small) return sm_fwd_prep(sh, X, A, scale, t_out, wsb, (hipStream_t)stream);
+    if (sh.small_fwd) return sm_fwd_prep(sh, X, A, scale, t_out, wsb, (hipStream_t)stream);
     return fwd_prep(sh, X, A, scale, t_out, wsb, (hipStream_t)stream);
 }
 
@@ -913,7 +925,7 @@ int r97q_qlinear_fwd_base(const R97qWeight* w, const uint16_t* X, int64_t T, con
     Shape sh = shape(T, w->rows, w->cols, rank);
     if (int e = settle(sh, true, true, workspace_bytes, workspace, who)) return e;
     uint8_t* wsb = static_cast<uint8_t*>(workspace);
-    if (sh.small) return sm_fwd_base(w, sh, B, Y, y_dtype, wsb, (hipStream_t)stream);
+    if (sh.small_fwd) return sm_fwd_base(w, sh, B, Y, y_dtype, wsb, (hipStream_t)stream);
     return fwd_base(w, sh, B, Y, y_dtype, wsb, (hipStream_t)stream);
 }
 
@@ -937,7 +949,7 @@ int r97q_qlinear_lora_fwd(const R97qWeight* w, const uint16_t* X, int64_t T, con
     if (int e = settle(sh, true, false, workspace_bytes, workspace, who)) return e;
     uint8_t* wsb = static_cast<uint8_t*>(workspace);
     const hipStream_t s = (hipStream_t)stream;
-    if (sh.small) return sm_fwd(w, sh, X, A, B, scale, Y, y_dtype, t_out, wsb, s);
+    if (sh.small_fwd) return sm_fwd(w, sh, X, A, B, scale, Y, y_dtype, t_out, wsb, s);
     if (int e = fwd_prep(sh, X, A, scale, t_out, wsb, s)) return e;
     return fwd_base(w, sh, B, Y, y_dtype, wsb, s);
 }
@@ -958,7 +970,7 @@ int r97q_lora_bwd_prep(int64_t T, int64_t N, int64_t K, const uint16_t* dY, cons
     Shape sh = shape(T, N, K, rank);
     if (int e = settle(sh, false, true, workspace_bytes, workspace, who)) return e;
     uint8_t* wsb = static_cast<uint8_t*>(workspace);
-    if (sh.small) return sm_bwd_prep(sh, dY, A, B, t, scale, wsb, (hipStream_t)stream);
+    if (sh.small_bwd) return sm_bwd_prep(sh, dY, A, B, t, scale, wsb, (hipStream_t)stream);
     return bwd_prep(sh, dY, A, B, t, scale, wsb, (hipStream_t)stream);
 }
 
@@ -977,7 +989,7 @@ int r97q_lora_bwd_grads(int64_t T, int64_t N, int64_t K, const uint16_t* X, cons
     Shape sh = shape(T, N, K, rank);
     if (int e = settle(sh, false, true, workspace_bytes, workspace, who)) return e;
     uint8_t* wsb = static_cast<uint8_t*>(workspace);
-    if (sh.small) return sm_bwd_grads(sh, X, dY, dA, dB, wsb, (hipStream_t)stream);
+    if (sh.small_bwd) return sm_bwd_grads(sh, X, dY, dA, dB, wsb, (hipStream_t)stream);
     return bwd_grads(sh, X, dY, dA, dB, wsb, (hipStream_t)stream);
 }
 
@@ -995,7 +1007,7 @@ int r97q_qlinear_dx_base(const R97qWeight* w, const uint16_t* dY, int64_t T, int
     Shape sh = shape(T, w->rows, w->cols, rank);
     if (int e = settle(sh, false, true, workspace_bytes, workspace, who)) return e;
     uint8_t* wsb = static_cast<uint8_t*>(workspace);
-    if (sh.small) return sm_dx_base(w, sh, dX, dx_dtype, dx_accumulate, wsb, (hipStream_t)stream);
+    if (sh.small_bwd) return sm_dx_base(w, sh, dX, dx_dtype, dx_accumulate, wsb, (hipStream_t)stream);
     return dx_base(w, sh, dX, dx_dtype, dx_accumulate, wsb, (hipStream_t)stream);
 }
 
@@ -1020,7 +1032,7 @@ int r97q_qlinear_lora_bwd(const R97qWeight* w, const uint16_t* X, const uint16_t
     if (int e = settle(sh, false, false, workspace_bytes, workspace, who)) return e;
     uint8_t* wsb = static_cast<uint8_t*>(workspace);
     const hipStream_t s = (hipStream_t)stream;
-    if (sh.small)
+    if (sh.small_bwd)
         return sm_bwd(w, sh, X, dY, A, B, scale, t, dX, dx_dtype, dx_accumulate, rank > 0 ? dA : nullptr,
                       rank > 0 ? dB : nullptr, wsb, s);
     if (int e = bwd_prep(sh, dY, A, B, t, scale, wsb, s)) return e;
@@ -1334,7 +1346,7 @@ int r97q_qlinear_lora_fwd_noalloc(const R97qWeight* w, const uint16_t* X, int64_
     }
     const Shape sh = shape(T, w->rows, w->cols, rank);
     // the few-token path's layout fits the array (kSmPartBytes); the others' runs the fused kernel
-    const bool small = sh.small && sm_ws(sh, true).fused <= kNoAllocScratchBytes;
+    const bool small = sh.small_fwd && sm_ws(sh, true).fused <= kNoAllocScratchBytes;
     const int64_t need = small ? sm_ws(sh, true).fused : fwd_ws(sh, true).total;
     if (need > kNoAllocScratchBytes) {
         set_error("%s: T %lld x K %lld at rank %d needs %lld workspace bytes, past the %lld this entry holds "

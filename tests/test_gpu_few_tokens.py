@@ -61,6 +61,8 @@ CASES = [
     (512, 4096, 4096, 32, 5, 256, False, False),
     (1000, 2048, 4096, 8, 4, 256, True, True),
     (1024, 256, 512, 32, 3, 256, False, False),  # the most tokens
+    (700, 6144, 128, 64, 5, 256, False, False),  # the forward past its line, the backward within
+    (846, 256, 6144, 8, 4, 128, True, False),    # and the other way round
 ]
 
 
