@@ -1001,11 +1001,13 @@ int64_t grad_blocks(int64_t C) { return (C + kGradCols - 1) / kGradCols; }
 int64_t grad_chunks(int64_t T, int64_t K, int64_t N, int r) {
     // Workgroups for the CUs over dA's and dB's column blocks, rounded down: one more than a CU holds at a
     // time makes the launch twice as long for the CU that takes it (dB over 12288 columns and 4096
-    // tokens at rank 16: 5 chunks, 240 workgroups, 31 us; 6 chunks, 288, 46). One workgroup a CU (two
-    // measured slower at ranks 8 to 32, 27-40%: the chunks' partial sums), two at rank 64, whose tiles
-    // are half as long (2048 + 8192 columns, 16384 tokens: 12 chunks 114 us, 6 chunks 130).
+    // tokens at rank 16: 5 chunks, 240 workgroups, 31 us; 6 chunks, 288, 46). One workgroup a CU: two
+    // measured slower at every rank (over random layers of 1025 to 16384 tokens the launch takes 1.1 to
+    // 1.4 times as long: the chunks' partial sums). Three quarters of one at rank 64, whose partial
+    // sums are the largest (2048 + 8192 columns, 16384 tokens: the launch 122 us, the backward 707; with 256
+    // workgroups 148 and 732, with 512 161 and 722).
     const int64_t cols = grad_blocks(K) + grad_blocks(N);
-    int64_t chunks = cols > 0 ? (r == 64 ? 512 : 256) / cols : 1;  // no columns: a size query's
+    int64_t chunks = cols > 0 ? (r == 64 ? 192 : 256) / cols : 1;  // no columns: a size query's
     const int64_t tiles = grad_ld(T) / 64;  // no chunk smaller than one 64-token tile
     if (chunks > tiles) chunks = tiles;
     return chunks < 1 ? 1 : chunks;
