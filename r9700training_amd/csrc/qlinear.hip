@@ -1255,8 +1255,11 @@ int r97q_lora_expand_bwd(int64_t T, int64_t N, const uint16_t* dY, const uint16_
     if (int e = check_ws(workspace_bytes, ws.total, workspace, who)) return e;
     uint8_t* wsb = static_cast<uint8_t*>(workspace);
     const hipStream_t s = (hipStream_t)stream;
-    if (few_adapter(T, rank) && reinterpret_cast<uintptr_t>(B) % 16 == 0) {
-        // two launches: dY.B over ranges, then t_cot and dB
+    // few tokens: two launches, dY.B over ranges, then t_cot and dB. t_cot alone is one launch below, whose
+    // waves walk N an eighth each: the faster one for few columns (720 tokens x 3456 at rank 16 7.2 us against
+    // 10.1 over ranges; 236 x 16256 at rank 32 31 against 10)
+    const bool ranges = dB || N >= (rank <= 16 ? 4096 : 2048) + 4 * T;
+    if (few_adapter(T, rank) && ranges && reinterpret_cast<uintptr_t>(B) % 16 == 0) {
         sm::Finish f{};
         f.T = T;
         f.rank = rank;

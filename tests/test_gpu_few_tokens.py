@@ -371,3 +371,27 @@ def test_shrink_dx_over_its_inputs(T, K, r):
         torch.cuda.synchronize()
         for a, b in zip(got, want):
             assert _rel(a, b) <= 2e-5, (over, _rel(a, b))
+
+
+@pytest.mark.parametrize("T,C,r", [(1, 2048, 32), (1, 2176, 32), (255, 5120, 16), (257, 5120, 16), (3, 128, 64)])
+def test_expand_one_output(T, C, r):
+    """The expand's adjoint asked for t_cot alone (on both sides of its line, 4096 or 2048 columns and 4 a
+    token) or dB alone, against float64 products with the bound above; dB alone the bits it has beside t_cot."""
+    from r9700training_amd import _ptr, _stream, check, lib
+    from r9700training_amd.qlinear import lora_expand_bwd
+
+    print(f"case expand one output T={T} C={C} r={r}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(T)
+    dY = torch.randn((T, C), generator=g, device="cuda").to(torch.bfloat16)
+    B = torch.randn((C, r), generator=g, device="cuda").to(torch.bfloat16)
+    t, u = torch.randn((T, r), generator=g, device="cuda"), torch.randn((T, r), generator=g, device="cuda")
+    cot, _ = lora_expand_bwd(dY, B, 2.0, t_cot=u.clone(), want_dB=False)
+    _, both = lora_expand_bwd(dY, B, 2.0, t=t)
+    L = lib()
+    ws = torch.empty(L.r97q_lora_expand_bwd_workspace_bytes(T, C, r), dtype=torch.uint8, device="cuda")
+    dB = torch.zeros((C, r), device="cuda")
+    check(L.r97q_lora_expand_bwd(T, C, _ptr(dY), _ptr(B), r, 2.0, _ptr(t), None, _ptr(dB), _ptr(ws), ws.numel(), _stream()),
+          "expand")
+    torch.cuda.synchronize()
+    assert _rel(cot, u.double() + 2.0 * (dY.double() @ B.double())) <= 2e-5
+    assert torch.equal(dB, both) and _rel(dB, 2.0 * (dY.double().T @ t.double())) <= 2e-5
