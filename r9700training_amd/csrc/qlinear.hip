@@ -1189,9 +1189,13 @@ int r97q_lora_shrink_bwd(int64_t T, int64_t K, const uint16_t* X, const uint16_t
     if (int e = check_ws(workspace_bytes, ws.total, workspace, who)) return e;
     uint8_t* wsb = static_cast<uint8_t*>(workspace);
     const hipStream_t s = (hipStream_t)stream;
-    // one launch: dX and dA from the f32 t_cot (a dX written over t_cot or A takes the launches below, which
-    // read both before they write it)
-    if (few_adapter(T, rank) && !overlap(dX, T * K * 4, t_cot, T * rank * 4) && !overlap(dX, T * K * 4, A, rank * K * 2)) {
+    // few tokens: one launch, dX and dA from the f32 t_cot. Not for a dX written over t_cot or A (the launches
+    // below read both before they write it), nor for dX alone where its f32 FMAs take longer than two launches
+    // with MFMAs do (346 x 14720 at rank 64 44 us against 30, 719 x 15104 at rank 32 38 against 35; 221 x 8448
+    // at rank 64 16 against 17)
+    const bool fmas = dA || T * K <= (rank == 64 ? 3000000 : 9000000);
+    if (few_adapter(T, rank) && fmas && !overlap(dX, T * K * 4, t_cot, T * rank * 4) &&
+        !overlap(dX, T * K * 4, A, rank * K * 2)) {
         sm::Finish f{};
         f.T = T;
         f.rank = rank;

@@ -395,3 +395,19 @@ def test_expand_one_output(T, C, r):
     torch.cuda.synchronize()
     assert _rel(cot, u.double() + 2.0 * (dY.double() @ B.double())) <= 2e-5
     assert torch.equal(dB, both) and _rel(dB, 2.0 * (dY.double().T @ t.double())) <= 2e-5
+
+
+@pytest.mark.parametrize("T,K,r", [(400, 7424, 64), (401, 7552, 64), (1000, 8960, 16), (1008, 8960, 16)])
+def test_shrink_dx_alone(T, K, r):
+    """The shrink's dX without dA on both sides of its line (3 and 9 million values), against float64
+    products with the bound above."""
+    from r9700training_amd.qlinear import lora_shrink_bwd
+
+    print(f"case shrink dX alone T={T} K={K} r={r}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(T)
+    u = torch.randn((T, r), generator=g, device="cuda")
+    A = torch.randn((r, K), generator=g, device="cuda").to(torch.bfloat16)
+    base = torch.randn((T, K), generator=g, device="cuda")
+    dX, _ = lora_shrink_bwd(None, A, u, dX=base.clone(), accumulate=True, want_dA=False)
+    torch.cuda.synchronize()
+    assert _rel(dX, base.double() + u.double() @ A.double()) <= 2e-5
