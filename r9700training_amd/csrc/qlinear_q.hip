@@ -340,9 +340,12 @@ __global__ __launch_bounds__(512) void qlinear_q_few_kernel(const Params p) {
 
 int launch_forward(const Params& p, hipStream_t s) {
     // Few tokens' tiles where they are at most four a CU (past that the 256 x 128 tile's reuse wins: 512
-    // tokens x 4096 outputs, 2048 tiles, 90 us against 55; 700 x 2048, 1408, 25 against 19); the codes
-    // on 16 bytes and the scales within the LDS, else the tile above.
-    if ((p.T + 31) / 32 * (p.N / 32) <= 1024 && p.K / kGroup <= kFewGroups &&
+    // tokens x 4096 outputs, 2048 tiles, 90 us against 55; 700 x 2048, 1408, 25 against 19), and half a CU
+    // for each group below eight, which leave waves idle (160 x 5504 over one group, 860 tiles, 16.4 us against
+    // 7.9; 285 x 1920 over three, 540, 12.2 against 10.6; 71 x 2432 over two, 228, 7.6 against 8.8); the
+    // codes on 16 bytes and the scales within the LDS, else the tile above.
+    const int64_t groups = p.K / kGroup;
+    if ((p.T + 31) / 32 * (p.N / 32) <= 128 * (groups < 8 ? groups : 8) && groups <= kFewGroups &&
         reinterpret_cast<uintptr_t>(p.a) % 16 == 0 && reinterpret_cast<uintptr_t>(p.codes) % 16 == 0) {
         hipLaunchKernelGGL(qlinear_q_few_kernel, dim3((unsigned)(p.N / 32), (unsigned)((p.T + 31) / 32)), dim3(512), 0, s, p);
         return launch_status("qlinear_q_few_kernel");

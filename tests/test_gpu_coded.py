@@ -282,11 +282,13 @@ def test_coded_shrink_da_over_t_cot(T, K, gw, r):
 
 
 @pytest.mark.parametrize("T,N,K,bf16", [(1, 128, 128, False), (31, 256, 640, True), (33, 384, 1152, False),
-                                        (100, 8192, 128, False), (130, 6528, 256, False), (129, 128, 4224, False)])
+                                        (100, 8192, 128, False), (130, 6528, 256, False), (129, 128, 4224, False),
+                                        (32, 4096, 128, False), (64, 4096, 256, True), (65, 4096, 256, False),
+                                        (100, 8192, 1024, False), (129, 8192, 1024, False)])
 def test_coded_forward_few_tokens(T, N, K, bf16):
-    """The coded forward on both sides of its few-token line (1024 tiles of 32 x 32: 100 x 8192 the last
-    of it, 130 x 6528 and beyond the larger tile) and off 16 bytes, against float64: the group sums are
-    exact, so what is left is the f32 fold over the groups (1e-6 relative) and a bf16 output's rounding."""
+    """The coded forward on both sides of its few-token line (128 tiles of 32 x 32 a group, up to 1024: 32 x
+    4096 over one, 64 x 4096 over two and 100 x 8192 over eight the last of it) and off 16 bytes, against
+    float64: the group sums are exact, so what is left is the f32 fold over the groups (1e-6 relative) and a bf16 output's rounding."""
     from r9700training_amd.qlinear import gemm_nt_q_fwd
 
     print(f"case coded forward T={T} N={N} K={K} bf16={bf16}", flush=True)
