@@ -243,9 +243,10 @@ int r97q_weight_from_decoded(const int8_t* codes, const uint16_t* scale, int64_t
  * the workspace (N*K*2 more bytes) and runs the product over the decoded tiles, the same values in
  * the same order (the results are the same bits); R97Q_DECODE_AUTO (the default) takes the second
  * from 16384 tokens on, and from 8192 for weights of 8M (2^23) values or more, and for calls of few
- * tokens (up to 128, and up to 1024 while the products are small) a path of two launches a direction
+ * tokens (up to 128, and up to 1024 while the products are small; not where a direction has many
+ * outputs over a short reduction) a path of two launches a direction
  * that deals each product's reduction over the CUs: the same decoded weights, the f32 sums in another
- * order. Process-wide; returns the previous mode, or -1 for an unknown one. The
+ * order. (Issued as the stages below, such a direction takes two launches more.) Process-wide; returns the previous mode, or -1 for an unknown one. The
  * workspace sizes below follow the mode in force when they are asked. */
 #define R97Q_DECODE_AUTO 0
 #define R97Q_DECODE_ONCE 1
@@ -342,7 +343,8 @@ int r97q_qlinear_dx_base(const R97qWeight* w, const uint16_t* dY, int64_t T, int
  * serving loops, harnesses that forbid hipMalloc). Same arguments, results and status as
  * r97q_qlinear_lora_fwd without the workspace pair; the workspace is a device array of the
  * library's own, one per GPU, of r97q_qlinear_lora_fwd_noalloc_max_bytes() bytes (48 MiB: T*K*2
- * plus T*r*4 and a little, e.g. T = K = 4096 at rank 16). A larger shape gets R97Q_EWORKSPACE.
+ * plus T*r*4 and a little, e.g. T = K = 4096 at rank 16; a call of few tokens, whose path needs its
+ * partial products, always fits). A larger shape gets R97Q_EWORKSPACE.
  * Calls that overlap on one GPU share that array and race: serialise them (one stream, or events). */
 int64_t r97q_qlinear_lora_fwd_noalloc_max_bytes(void);
 int r97q_qlinear_lora_fwd_noalloc(const R97qWeight* w, const uint16_t* X, int64_t T, const uint16_t* A,

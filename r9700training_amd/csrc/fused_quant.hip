@@ -338,8 +338,8 @@ __device__ __forceinline__ double sigm_lane(double x) {
 
 // The gates, flat over the units. Bound by memory in the adjoint and by the f64 instructions (the
 // exponential, the division, the butterflies) in the forward. Measured at 4096 x 17408 bf16, silu_mul,
-// group 128: forward 253 us (2.0 TB/s) and adjoint 377 us (5.3 TB/s), against 334 and 1069 us for one
-// column a lane and LDS permutes.
+// group 128, with y and its cotangent: forward 222 us (2.3 TB/s) and adjoint 368 us (5.4 TB/s), against
+// 338 and 1074 us for one column a lane and LDS permutes.
 template <int PART, class T>
 __global__ __launch_bounds__(lanes::kThreads) void lane_fwd_kernel(const LaneArgs q) {
     const int64_t u = (int64_t)blockIdx.x * lanes::kThreads + threadIdx.x;
@@ -405,9 +405,11 @@ __global__ __launch_bounds__(lanes::kThreads) void lane_bwd_kernel(const LaneArg
 }
 
 // The norm: a workgroup a row, as many threads as the row has units up to 1024, IT units a thread,
-// the row held in registers from its one read to the last use. Measured at 64 x 5120 f32, group 128:
-// forward 6.0 us and adjoint 7.9 us, against 19.6 and 52.1 us for four waves walking the row three
-// times.
+// the row held from its one read to the last use -- in registers, but for the adjoint past 8192 columns,
+// which spills (17 registers a lane at IT 2, 78 at IT 3). Measured with group 128 (y and its cotangent
+// written and read), against four waves walking the row three times: 64 x 5120 f32 forward 6.0 us and
+// adjoint 7.8, against 21 and 58; 64 x 12288 8.2 and 15, against 48 and 133; 64 x 17408 10 and 31, against 67
+// and 186; 2048 x 17408 bf16 83 and 378, against 177 and 961.
 constexpr int kNormMaxIt = 3;
 
 __device__ double row_sum(double s, double* red) {

@@ -34,25 +34,20 @@ __device__ __forceinline__ uint32_t other(uint32_t x) {
     return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x128, 0xF, 0xF, true);  // the row rotated by 8
 }
 
-// (lower, upper) of the pair of lanes H apart, in both of them
+// (lower, upper) of the pair of lanes H apart (16 or 32), in both of them
 template <int H>
-__device__ __forceinline__ void pair(double v, bool upper, double& lo, double& hi) {
+__device__ __forceinline__ void pair(double v, double& lo, double& hi) {
+    static_assert(H == 16 || H == 32, "the row swaps");
     const uint64_t b = __builtin_bit_cast(uint64_t, v);
     const uint32_t x = (uint32_t)b, y = (uint32_t)(b >> 32);
-    if constexpr (H < 16) {
-        const double o = __builtin_bit_cast(double, (uint64_t)other<H>(y) << 32 | other<H>(x));
-        lo = upper ? o : v;
-        hi = upper ? v : o;
-    } else {
-        // the swap exchanges the odd 16-lane rows (H 16) or the upper half (H 32) of its first operand
-        // with the even rows (the lower half) of its second: given x twice, the lower and the upper
-        const auto sx = H == 16 ? __builtin_amdgcn_permlane16_swap(x, x, false, false)
-                                : __builtin_amdgcn_permlane32_swap(x, x, false, false);
-        const auto sy = H == 16 ? __builtin_amdgcn_permlane16_swap(y, y, false, false)
-                                : __builtin_amdgcn_permlane32_swap(y, y, false, false);
-        lo = __builtin_bit_cast(double, (uint64_t)sy[0] << 32 | sx[0]);
-        hi = __builtin_bit_cast(double, (uint64_t)sy[1] << 32 | sx[1]);
-    }
+    // the swap exchanges the odd 16-lane rows (H 16) or the upper half (H 32) of its first operand
+    // with the even rows (the lower half) of its second: given x twice, the lower and the upper
+    const auto sx = H == 16 ? __builtin_amdgcn_permlane16_swap(x, x, false, false)
+                            : __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    const auto sy = H == 16 ? __builtin_amdgcn_permlane16_swap(y, y, false, false)
+                            : __builtin_amdgcn_permlane32_swap(y, y, false, false);
+    lo = __builtin_bit_cast(double, (uint64_t)sy[0] << 32 | sx[0]);
+    hi = __builtin_bit_cast(double, (uint64_t)sy[1] << 32 | sx[1]);
 }
 
 // one stage between lanes H apart: lo + hi in the lower lane, lo - hi in the upper. For H < 16 the
@@ -71,7 +66,7 @@ __device__ __forceinline__ void stage(double (&v)[kV], int lane) {
             v[k] = __builtin_bit_cast(double, o) + negated(v[k]);
         } else {
             double lo, hi;
-            pair<H>(v[k], false, lo, hi);
+            pair<H>(v[k], lo, hi);
             v[k] = lo + negated(hi);
         }
     }
@@ -104,7 +99,7 @@ __device__ __forceinline__ double max_with(double m) {
         lo = m;
         hi = __builtin_bit_cast(double, (uint64_t)other<H>((uint32_t)(b >> 32)) << 32 | other<H>((uint32_t)b));
     } else {
-        pair<H>(m, false, lo, hi);
+        pair<H>(m, lo, hi);
     }
     return fmax(lo, hi);
 }

@@ -60,8 +60,8 @@ struct Shape {
 //     for 2048 x 2048 (0.229 ms against 0.214);
 //   - it wins at 32 and 64 panels (4096 x 4096 at 16384 tokens: 1.21 ms against 1.27; C5's 32768
 //     tokens: the 24-layer step 182 ms against 191).
-// r97q_set_decode_once overrides the choice; the entry that allocates nothing always runs the
-// fused kernel.
+// r97q_set_decode_once overrides the choice; the entry that allocates nothing never decodes once: it
+// takes the few-token path below or the fused kernel.
 constexpr int64_t kDecodeOnceMinT = 32 * rt::kBM;          // any weight from 16384 tokens
 constexpr int64_t kDecodeOnceMinTLarge = 16 * rt::kBM;     // weights of kDecodeOnceLarge values from 8192
 constexpr int64_t kDecodeOnceLarge = int64_t(1) << 23;

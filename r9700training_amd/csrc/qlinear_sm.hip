@@ -314,7 +314,7 @@ __device__ __forceinline__ void product_item(const Params& p, uint8_t* tiles, ui
 #pragma unroll
     for (int i = 0; i < kRing; ++i) fetch(s0 + i, wd[i], tk[i]);
     fill(wd[0], tk[0], toks, tiles);
-    // step s + I: the loads of step s + I + 4 on their way, the step's products from one LDS slot beside
+    // step s + I: the loads of step s + I + kRing on their way, the step's products from one LDS slot beside
     // the next step's decode into the other
     auto multiply = [&](const uint8_t* tok, const uint8_t* cur) {
 #pragma unroll

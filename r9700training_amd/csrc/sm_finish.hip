@@ -6,9 +6,10 @@
 //   dX[m][k] (+)= sum_z part[z][m][k] + sum_j u[m][j] A[j][k]   u = dt                   (backward)
 //   dA[j][k] += sum_m u[m][j] X[m][k]      dB[n][j] += sum_m s t[m][j] dY[m][n]
 //
-// The adapter's sums run in f32 FMAs over the exact f32 u and t (the larger calls' MFMAs take them as
-// two bf16 halves): at the token counts of this path they are a few microseconds of the chip's vector
-// rate, less than the staging MFMAs would need. All sums run in an order that the shape alone fixes.
+// The adapter's sums run over the exact f32 u and t (the larger calls' bf16 MFMAs take them as two
+// halves): the up-projection in f32 FMAs, a few microseconds of the chip's vector rate at the token counts
+// of this path, less than staging it for MFMAs would need; the factor gradients on the f32 MFMAs
+// (grad_item). All sums run in an order that the shape alone fixes.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
